@@ -1,0 +1,571 @@
+// The tile that the prefill / training GEMM of the packed weight
+// (nf4_mfma.hip) and the dense matmul (dense_matmul.hip) share:
+//
+//     result [rows, columns] = left [rows, K] . right [K, columns]
+//
+// in fp32 on the bf16 matrix instructions.
+//
+// The product.  An fp32 value is the exact sum of three bf16 values (8 + 8 + 8
+// significand bits): hi = the value rounded to bf16 (right operand: cut), mid =
+// the rest rounded to bf16, lo = what then remains, which has at most eight
+// significant bits and is exact.  left . right is then six products on
+// v_mfma_f32_32x32x16_bf16, all added into fp32 accumulators,
+//     hi.hi + (hi.mid + mid.hi) + (hi.lo + mid.mid + lo.hi),
+// each exact before its addition.  What is left out, mid.lo + lo.mid + lo.lo,
+// is at most 2^-23 of a term and without bias (a single rounding of the term
+// is 2^-24), far below the roundings of the sum; and there are fewer of those,
+// as a matrix instruction takes sixteen contraction values instead of two.
+// Against sums in 64 bits at 2048 rows of 11008 x 4096 the forward measures
+// 2.5e-7 (2-norm, relative) where v_mfma_f32_32x32x2_f32 over the same values
+// measured 2.8e-7; all nine products measure the same 2.5e-7 (and 0.43 ms where
+// six take 0.33).
+//
+// What bounds it: the device's power.  v_mfma_f32_32x32x16_bf16 alone, on
+// normally distributed values, runs at 1840 TFLOP/s (1.8 GHz), i.e. 307
+// TFLOP/s of six products each; this tile reaches 205-218 TFLOP/s at 1.85 GHz
+// (2048 rows of 4096 x 4096: 0.32 ms; the fp32 instruction: 0.53 ms).  One
+// tile on an otherwise idle device takes 225 us of those 320 us.
+//
+// Infinities: hi + mid + lo of an infinite value would be a NaN, so it is
+// passed on as (0, 0, infinity): lo meets the other operand's hi alone, and
+// the sum is the infinity (or the NaN of infinity times zero) that fp32
+// arithmetic gives.  bf16 keeps fp32's exponent range and the matrix cores take
+// subnormal bf16 values as they are, so only values under 2^-110 have bits that
+// fall below bf16's smallest step, 2^-133, and are lost.
+#pragma once
+
+#include "gemv_shared.hpp"
+#include "kernels.hpp"
+
+#include <cstddef>
+#include <cstdint>
+
+namespace rthip {
+namespace {
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kPlanes = 3;        // hi, mid, lo
+constexpr int kTileN = 128;       // output columns per workgroup
+constexpr unsigned kFragmentBytes = 1024;  // 32 rows x 16 contraction values
+constexpr unsigned kFlushValues = 256;  // contraction values per accumulation
+constexpr unsigned kOutside = 0xFFFFFFFFU;  // past every descriptor's extent
+
+// Two values as three bf16 pairs (the first value in the low half).
+struct SplitPair {
+    unsigned hi;
+    unsigned mid;
+    unsigned lo;
+};
+
+__device__ __forceinline__ unsigned round_pair(float a, float b) {
+    return __builtin_bit_cast(
+        unsigned, __builtin_convertvector((floatx2{a, b}), bf16x2));
+}
+__device__ __forceinline__ unsigned cut_pair(float a, float b) {
+    return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b),
+                                 __builtin_bit_cast(unsigned, a),
+                                 0x07060302U);
+}
+__device__ __forceinline__ float low_value(unsigned pair) {
+    return __builtin_bit_cast(float, pair << 16);
+}
+__device__ __forceinline__ float high_value(unsigned pair) {
+    return __builtin_bit_cast(float, pair & 0xFFFF0000U);
+}
+
+// kRounded: magnitudes from kRoundsToInfinity on must not occur.
+constexpr float kRoundsToInfinity = 0x1.FFp+127F;
+template <bool kRounded>
+__device__ __forceinline__ SplitPair split_pair(float a, float b) {
+    SplitPair out;
+    float a_rest;
+    float b_rest;
+    if constexpr (kRounded) {
+        out.hi = round_pair(a, b);
+        a_rest = a - low_value(out.hi);
+        b_rest = b - high_value(out.hi);
+    } else {
+        out.hi = cut_pair(a, b);
+        a_rest = a - high_value(__builtin_bit_cast(unsigned, a));
+        b_rest = b - high_value(__builtin_bit_cast(unsigned, b));
+    }
+    out.mid = round_pair(a_rest, b_rest);
+    out.lo =
+        cut_pair(a_rest - low_value(out.mid), b_rest - high_value(out.mid));
+    return out;
+}
+
+// The same for any values.
+__device__ __forceinline__ SplitPair split_any_pair(float a, float b) {
+    SplitPair out = split_pair<false>(a, b);
+    if (__builtin_isinf(a)) {
+        out.hi &= 0xFFFF0000U;
+        out.mid &= 0xFFFF0000U;
+        out.lo = (out.lo & 0xFFFF0000U) |
+                       (__builtin_bit_cast(unsigned, a) >> 16);
+    }
+    if (__builtin_isinf(b)) {
+        out.hi &= 0xFFFFU;
+        out.mid &= 0xFFFFU;
+        out.lo = (out.lo & 0xFFFFU) |
+                       (__builtin_bit_cast(unsigned, b) & 0xFFFF0000U);
+    }
+    return out;
+}
+
+// max(largest, |a|, |b|) in one instruction
+__device__ __forceinline__ float raise_magnitude(float largest, float a,
+                                                 float b) {
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(largest) : "v"(a), "v"(b));
+    return largest;
+}
+
+// The two tile shapes.  Tall: 256 output rows, eight wavefronts, steps of 32
+// contraction values, one workgroup per compute unit: an element of the right
+// operand is decoded and split once per 256 rows.  Otherwise 128 rows, four
+// wavefronts, steps of 16, two workgroups per compute unit.  A wavefront owns
+// 64 x 64 outputs in both, as 2 x 2 blocks of the 32 x 32 x 16 instruction.
+template <bool kTall>
+struct Tile {
+    static constexpr int kThreads = kTall ? 512 : 256;
+    static constexpr int kTileM = kTall ? 256 : 128;  // output rows
+    static constexpr int kStep = kTall ? 32 : 16;     // contraction per step
+    static constexpr int kSlices = kStep / 16;  // matrix instructions' K
+    static constexpr int kOctets = kStep / 8;   // a lane's eight values
+    static constexpr int kWorkgroupsPerUnit = kTall ? 1 : 2;
+    // workgroups the device holds at once
+    static constexpr unsigned kPlaces = kTall ? 256 : 512;
+    // rows of the left operand per pass of the workgroup (a float4 per thread)
+    static constexpr int kPassRows = kThreads / (kStep / 4);
+    static constexpr int kPasses = kTileM / kPassRows;
+    static constexpr unsigned kBlockBytes =
+        kSlices * kPlanes * kFragmentBytes;  // 32 rows or columns
+    static constexpr unsigned kLeftBytes = kTileM / 32 * kBlockBytes;
+    static constexpr unsigned kBufferBytes =
+        kLeftBytes + kTileN / 32 * kBlockBytes;
+    // LDS of a workgroup: two buffers of both tiles
+    static constexpr std::size_t kTileBytes = std::size_t{2} * kBufferBytes;
+};
+
+// Where the eight contraction values [8 * octet, 8 * octet + 8) of a row (or
+// column) of the tile lie in LDS, in bytes, plane 0.  The tile is kept as the
+// matrix instruction reads it: per 32 rows, per 16 contraction values, per
+// plane one kilobyte, a lane's sixteen bytes after the other (lane = row % 32
+// + 32 * (octet % 2)), so that a fragment is one conflict-free ds_read_b128.
+// The XOR turns the rows so that the writes -- neighbouring lanes hold
+// neighbouring octets of a row -- spread over all banks as well.
+template <bool kTall>
+__device__ __forceinline__ unsigned tile_address(unsigned row,
+                                                 unsigned octet) {
+    const unsigned half = octet % 2;
+    const unsigned slice = octet / 2;
+    const unsigned turned =
+        (row % 32) ^ (kTall ? 2 * half + 4 * slice : 4 * half);
+    return (row / 32) * Tile<kTall>::kBlockBytes +
+           slice * (kPlanes * kFragmentBytes) + half * 512 + turned * 16;
+}
+
+// Splits eight values and writes them.
+template <bool kCareful>
+__device__ __forceinline__ void store_octet(char* target,
+                                            const float (&values)[8]) {
+    uintx4 planes[kPlanes];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const SplitPair pair =
+            kCareful
+                ? split_any_pair(values[2 * p], values[2 * p + 1])
+                : split_pair<false>(values[2 * p], values[2 * p + 1]);
+        planes[0][p] = pair.hi;
+        planes[1][p] = pair.mid;
+        planes[2][p] = pair.lo;
+    }
+#pragma unroll
+    for (int p = 0; p < kPlanes; ++p) {
+        *reinterpret_cast<uintx4*>(target + p * kFragmentBytes) = planes[p];
+    }
+}
+
+// The left operand: fp32 rows of `width` contraction values.  Thread t takes
+// float4 t % (kStep / 4) of rows t / (kStep / 4) + kPassRows * pass.  Every
+// load is a buffer load whose per-lane offset is fixed for the whole segment
+// and whose scalar offset advances with the step; rows past the last one are
+// past the descriptor's extent, where the hardware returns zeros.
+template <bool kTall, bool kRagged>
+class LeftTile {
+public:
+    __device__ __forceinline__ LeftTile(const float* left, unsigned width,
+                                        unsigned row0, unsigned rows)
+        : width_(width),
+          column_((threadIdx.x % kPerRow) * 4),
+          buffer_(make_buffer(
+              left + static_cast<std::size_t>(row0) * width,
+              static_cast<unsigned>(
+                  min(rows - row0,
+                      static_cast<unsigned>(Tile<kTall>::kTileM)) *
+                  static_cast<std::size_t>(width) * sizeof(float)))) {
+#pragma unroll
+        for (int pass = 0; pass < Tile<kTall>::kPasses; ++pass) {
+            const unsigned row =
+                threadIdx.x / kPerRow + Tile<kTall>::kPassRows * pass;
+            lane_[pass] = static_cast<unsigned>((row * width + column_) *
+                                                sizeof(float));
+        }
+        target_ = tile_address<kTall>(threadIdx.x / kPerRow, column_ / 8) +
+                  (column_ / 4) % 2 * 8;
+    }
+
+    // Requests pass `pass` of the step that starts at k.
+    __device__ __forceinline__ void load(unsigned k, int pass) {
+        const unsigned step = k * static_cast<unsigned>(sizeof(float));
+        if constexpr (kRagged) {
+            // the row ends inside this step: value by value
+            if (k + Tile<kTall>::kStep > width_) {  // uniform
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    values_[pass][e] = __builtin_bit_cast(
+                        float, __builtin_amdgcn_raw_buffer_load_b32(
+                                   buffer_,
+                                   k + column_ + e < width_
+                                       ? lane_[pass] + 4 * e
+                                       : kOutside,
+                                   step, 0));
+                }
+                return;
+            }
+        }
+        values_[pass] = __builtin_bit_cast(
+            floatx4, __builtin_amdgcn_raw_buffer_load_b128(
+                         buffer_, lane_[pass], step, 0));
+    }
+
+    // Splits pass `pass` and writes it.  kCareful: any value; otherwise
+    // `largest` is raised to the largest magnitude met, by which the caller
+    // learns of values that may not be rounded.
+    template <bool kCareful>
+    __device__ __forceinline__ void store(char* tile, int pass,
+                                          float& largest) const {
+        const floatx4 v = values_[pass];
+        SplitPair first;
+        SplitPair second;
+        if constexpr (kCareful) {
+            first = split_any_pair(v.x, v.y);
+            second = split_any_pair(v.z, v.w);
+        } else {
+            first = split_pair<true>(v.x, v.y);
+            second = split_pair<true>(v.z, v.w);
+            largest = raise_magnitude(largest, v.x, v.y);
+            largest = raise_magnitude(largest, v.z, v.w);
+        }
+        char* const target =
+            tile + target_ +
+            pass * (Tile<kTall>::kPassRows / 32) * Tile<kTall>::kBlockBytes;
+        *reinterpret_cast<uintx2*>(target) = uintx2{first.hi, second.hi};
+        *reinterpret_cast<uintx2*>(target + kFragmentBytes) =
+            uintx2{first.mid, second.mid};
+        *reinterpret_cast<uintx2*>(target + 2 * kFragmentBytes) =
+            uintx2{first.lo, second.lo};
+    }
+
+private:
+    static constexpr unsigned kPerRow = Tile<kTall>::kStep / 4;
+    static_assert(Tile<kTall>::kPassRows % 32 == 0);
+    unsigned width_;
+    unsigned column_;
+    __amdgpu_buffer_rsrc_t buffer_;
+    unsigned lane_[Tile<kTall>::kPasses];
+    unsigned target_;
+    floatx4 values_[Tile<kTall>::kPasses];
+};
+
+// Accumulators of a wavefront's 64 x 64 outputs.  Two levels: the matrix
+// instructions add into `acc` for 256 contraction values, then `acc` is folded
+// into `total` and cleared.  One long fp32 chain over K = 11008 drifts about as
+// far as the CPU's sequential sum (~1e-5 of an output's standard deviation);
+// chains of 256 stay an order of magnitude below that.
+struct Accumulators {
+    floatx16 acc[2][2];
+    floatx16 total[2][2];
+
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    acc[i][j][e] = 0.0F;
+                    total[i][j][e] = 0.0F;
+                }
+            }
+        }
+    }
+    // total += factor * acc; acc = 0
+    __device__ __forceinline__ void fold(float factor) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    total[i][j][e] += factor * acc[i][j][e];
+                    acc[i][j][e] = 0.0F;
+                }
+            }
+        }
+    }
+    __device__ __forceinline__ void fold() {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    total[i][j][e] += acc[i][j][e];
+                    acc[i][j][e] = 0.0F;
+                }
+            }
+        }
+    }
+};
+
+// A wavefront's operands of one slice (16 contraction values): 64 rows of the
+// left tile and 64 columns of the right tile.
+template <bool kTall>
+class Fragments {
+public:
+    // tiles: a buffer; the slice of it that the fragments start from
+    __device__ __forceinline__ void load(const char* tiles, int slice) {
+        load_left(tiles, slice, 1);
+        load_right(tiles, slice, 1);
+        load_left(tiles, slice, 2);
+        load_right(tiles, slice, 2);
+        load_left(tiles, slice, 0);
+        load_right(tiles, slice, 0);
+    }
+    // The slice's six products, 24 matrix instructions.  An operand plane is
+    // replaced by that of the next slice (`next_slice` of the buffer at
+    // `next`) as soon as its last product is issued, so that the next slice
+    // starts without waiting for LDS.  between(group) is called after each
+    // group of four instructions; the replacements start after the third.
+    template <class Between>
+    __device__ __forceinline__ void multiply(Accumulators& sums,
+                                             const char* next, int next_slice,
+                                             const Between& between) {
+        product(sums, 1, 1);
+        between(0);
+        product(sums, 1, 0);
+        between(1);
+        product(sums, 0, 1);
+        between(2);
+        load_left(next, next_slice, 1);
+        load_right(next, next_slice, 1);
+        product(sums, 2, 0);
+        load_left(next, next_slice, 2);
+        between(3);
+        product(sums, 0, 2);
+        load_right(next, next_slice, 2);
+        between(4);
+        product(sums, 0, 0);
+        load_left(next, next_slice, 0);
+        load_right(next, next_slice, 0);
+        between(5);
+    }
+
+private:
+    __device__ __forceinline__ static unsigned octet(int slice) {
+        return 2 * slice + threadIdx.x % 64 / 32;
+    }
+    __device__ __forceinline__ void load_left(const char* tiles, int slice,
+                                              int plane) {
+        const unsigned row =
+            (threadIdx.x / 128) * 64 + threadIdx.x % 32;
+        const char* const source = tiles +
+                                   tile_address<kTall>(row, octet(slice)) +
+                                   plane * kFragmentBytes;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            left_[i][plane] = *reinterpret_cast<const bf16x8*>(
+                source + i * Tile<kTall>::kBlockBytes);
+        }
+    }
+    __device__ __forceinline__ void load_right(const char* tiles, int slice,
+                                               int plane) {
+        const unsigned column =
+            (threadIdx.x / 64 % 2) * 64 + threadIdx.x % 32;
+        const char* const source = tiles + Tile<kTall>::kLeftBytes +
+                                   tile_address<kTall>(column, octet(slice)) +
+                                   plane * kFragmentBytes;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            right_[j][plane] = *reinterpret_cast<const bf16x8*>(
+                source + j * Tile<kTall>::kBlockBytes);
+        }
+    }
+    __device__ __forceinline__ void product(Accumulators& sums, int left,
+                                            int right) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                sums.acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    left_[i][left], right_[j][right], sums.acc[i][j], 0, 0,
+                    0);
+            }
+        }
+    }
+    bf16x8 left_[2][kPlanes];
+    bf16x8 right_[2][kPlanes];
+};
+
+// Contraction steps [k_begin, k_end) (multiples of the step, the end possibly
+// past the operands' last value) of one output tile.  `tiles` is the
+// workgroup's LDS: two buffers.  A step multiplies from one buffer while the
+// next step's tiles -- whose operands are in registers by then -- are split
+// and written into the other, a piece after each group of matrix
+// instructions, and the operands of the step after that are requested into
+// the freed registers.  The step's
+// one barrier stands in the middle of its last slice, whose operands are in
+// registers: behind it the other buffer is complete, this one may be
+// overwritten, and half a slice of matrix instructions covers the first reads
+// of the next step.  (The last step splits and writes what lies past the end,
+// which is never used; the descriptors' extents keep the loads inside the
+// operands.)  Returns the largest magnitude of the left operand that the
+// thread met (kCareful: zero).
+template <bool kTall, bool kCareful, class Left, class Right>
+__device__ __forceinline__ float multiply_steps(Accumulators& sums, Left& left,
+                                                Right& right, char* tiles,
+                                                unsigned k_begin,
+                                                unsigned k_end) {
+    constexpr unsigned kStep = Tile<kTall>::kStep;
+    constexpr int kPasses = Tile<kTall>::kPasses;
+    constexpr int kSlices = Tile<kTall>::kSlices;
+    constexpr unsigned kLeftBytes = Tile<kTall>::kLeftBytes;
+    constexpr unsigned kBufferBytes = Tile<kTall>::kBufferBytes;
+    float largest = 0.0F;
+    const auto load_left = [&](unsigned k) {
+#pragma unroll
+        for (int pass = 0; pass < kPasses; ++pass) {
+            left.load(k, pass);
+        }
+    };
+    right.prime(k_begin);
+    load_left(k_begin);
+    right.load(k_begin);
+    __syncthreads();  // nobody still reads the tiles of an earlier segment
+#pragma unroll
+    for (int pass = 0; pass < kPasses; ++pass) {
+        left.template store<kCareful>(tiles, pass, largest);
+    }
+    right.store(tiles + kLeftBytes);
+    load_left(k_begin + kStep);
+    right.load(k_begin + kStep);
+    __syncthreads();
+
+    Fragments<kTall> fragments;
+    fragments.load(tiles, 0);
+    unsigned buffer = 0;
+    for (unsigned k0 = k_begin; k0 < k_end;) {
+        const unsigned fold_at = min(k0 + kFlushValues, k_end);
+        do {
+            const char* const current = tiles + buffer * kBufferBytes;
+            char* const target = tiles + (buffer ^ 1U) * kBufferBytes;
+            if constexpr (kSlices == 2) {
+                fragments.multiply(sums, current, 1, [&](int group) {
+                    if (group == 0) {
+                        right.store(target + kLeftBytes);
+                        right.load(k0 + 2 * kStep);
+                    } else if (group <= kPasses) {
+                        left.template store<kCareful>(target, group - 1,
+                                                      largest);
+                    } else {
+                        load_left(k0 + 2 * kStep);
+                    }
+                });
+            }
+            fragments.multiply(sums, target, 0, [&](int group) {
+                if constexpr (kSlices == 1) {
+                    if (group == 0) {
+                        right.store(target + kLeftBytes);
+                        right.load(k0 + 2 * kStep);
+                    } else if (group <= kPasses) {
+                        left.template store<kCareful>(target, group - 1,
+                                                      largest);
+                    } else if (group == 3) {
+                        load_left(k0 + 2 * kStep);
+                    }
+                }
+                if (group == 2) {
+                    __syncthreads();
+                }
+            });
+            buffer ^= 1U;
+            k0 += kStep;
+        } while (k0 < fold_at);
+        sums.fold();
+    }
+    __syncthreads();  // the tiles have been read
+    return largest;
+}
+
+// The whole of it: a second, careful pass where a value was infinite, or so
+// large that rounding to bf16 made it so.
+template <bool kTall, class Left, class Right>
+__device__ __forceinline__ void multiply_tile(Accumulators& sums, Left& left,
+                                              Right& right, char* tiles,
+                                              unsigned k_begin,
+                                              unsigned k_end) {
+    sums.clear();
+    const float largest = multiply_steps<kTall, false>(sums, left, right,
+                                                       tiles, k_begin, k_end);
+    if (__syncthreads_or(largest >= kRoundsToInfinity)) {
+        sums.clear();
+        multiply_steps<kTall, true>(sums, left, right, tiles, k_begin, k_end);
+    }
+}
+
+// Calls store(row in tile, column in tile, value) for every output of the
+// lane.  Accumulator element e of lane l is output row 8 * (e / 4) +
+// 4 * (l / 32) + e % 4, column l % 32 of its 32 x 32 block.
+template <class Store>
+__device__ __forceinline__ void for_each_output(const Accumulators& sums,
+                                                const Store& store) {
+    const unsigned lane = threadIdx.x % 64;
+    const unsigned wave = threadIdx.x / 64;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const unsigned column = (wave % 2) * 64 + j * 32 + lane % 32;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const unsigned row = (wave / 2) * 64 + i * 32 + 8 * (e / 4) +
+                                     4 * (lane / 32) + e % 4;
+                store(row, column, sums.total[i][j][e]);
+            }
+        }
+    }
+}
+
+// Workgroups are started on the eight XCDs in turn; block b of a launch of
+// `count` takes this item instead, so that every XCD (its own L2) gets a
+// contiguous run of the items.
+__device__ __forceinline__ unsigned xcd_contiguous(unsigned block,
+                                                   unsigned count) {
+    constexpr unsigned kXcds = 8;
+    const unsigned xcd = block % kXcds;
+    const unsigned quotient = count / kXcds;
+    const unsigned remainder = count % kXcds;
+    return xcd * quotient + min(xcd, remainder) + block / kXcds;
+}
+
+}  // namespace
+}  // namespace rthip

@@ -1,0 +1,102 @@
+"""The tiled products that split fp32 values into three bf16 values
+(riftco-transformer_amd/csrc/split_tile.hpp), at the edges of their tiles and of
+the fp32 range.
+
+Bounds.  A product keeps all but 2^-23 of itself; its sum runs in fp32 chains
+of 256 values.  The suite's bar of 1e-5 of a K-normalised output leaves a factor
+of ten over the chains' rounding.  A row of x with a single one in it meets no
+rounding at all: hi + mid + lo of a weight is the weight."""
+import numpy as np
+import pytest
+
+import helpers
+
+pytestmark = pytest.mark.gpu
+
+TOLERANCE = 1.0e-5
+
+
+def packed(package, oracle, gpu, out_w, in_w, block, nested, seed):
+    weight = oracle.quantize(helpers.normal(seed, (out_w, in_w), 0.02), block,
+                             nested, 32)
+    device = gpu.upload_weight(
+        out_w, in_w, block, weight.codes, fp32_scales=weight.fp32_scales,
+        scale_codes=weight.scale_codes, second_level=weight.second_level,
+        second_level_block=weight.second_level_block, offset=weight.offset)
+    return device, oracle.dequantize(weight)
+
+
+def run(gpu, function, activations, weight, package):
+    import torch
+    out = function(torch.from_numpy(activations).cuda(), weight,
+                   algorithm=package.ALGORITHM_MFMA)
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("nested", [False, True])
+@pytest.mark.parametrize("rows,out_w,in_w,block", [
+    (1, 32, 32, 32),          # one step, one octet's block
+    (127, 96, 64, 32),        # a row short of the 128-row tile
+    (129, 160, 96, 32),       # 256-row tile, one row past its half
+    (256, 128, 256, 64),      # whole tiles, one fold
+    (257, 352, 288, 32),      # one row past the 256-row tile; fold + 1 step
+    (300, 4064, 1056, 32),    # tiles dealt in runs
+])
+def test_tile_edges(gpu, package, oracle, rows, out_w, in_w, block, nested):
+    weight, dense = packed(package, oracle, gpu, out_w, in_w, block, nested,
+                           901)
+    unit = helpers.rms(dense)
+    for function, width, product in (
+            (gpu.linear_forward, in_w, helpers.exact_forward),
+            (gpu.linear_input_backward, out_w, helpers.exact_input_backward)):
+        values = helpers.normal(902, (rows, width), 1.0)
+        got = run(gpu, function, values, weight, package)
+        error = helpers.normalized_error(got, product(values, dense), width,
+                                         1.0, unit)
+        assert error <= TOLERANCE, f"{function.__name__}: {error:.3g}"
+
+
+@pytest.mark.parametrize("rows", [128, 256])
+def test_single_ones_return_the_weight(gpu, package, oracle, rows):
+    weight, dense = packed(package, oracle, gpu, 256, 256, 64, True, 903)
+    ones = np.eye(rows, 256, dtype=np.float32)
+    helpers.assert_bit_equal(
+        run(gpu, gpu.linear_forward, ones, weight, package), dense.T[:rows])
+    helpers.assert_bit_equal(
+        run(gpu, gpu.linear_input_backward, ones, weight, package),
+        dense[:rows])
+
+
+@pytest.mark.parametrize("rows", [100, 200])
+def test_infinite_and_huge_values(gpu, package, oracle, rows):
+    """Rows with values that are infinite, not a number, or round to infinity
+    in bf16: the same outputs are infinite or not a number as in 64 bits, and
+    the other rows are what they are without them."""
+    weight, dense = packed(package, oracle, gpu, 256, 256, 64, False, 904)
+    plain = helpers.normal(905, (rows, 256), 1.0)
+    special = plain.copy()
+    special[3, 7] = np.inf
+    special[5, 200] = -np.inf
+    special[8, 100] = np.nan
+    special[40, 31] = np.float32(3.4028e38)
+    touched = [3, 5, 8, 40]
+    others = np.setdiff1d(np.arange(rows), touched)
+    for function, product in (
+            (gpu.linear_forward, helpers.exact_forward),
+            (gpu.linear_input_backward, helpers.exact_input_backward)):
+        got = run(gpu, function, special, weight, package)
+        with np.errstate(invalid="ignore", over="ignore"):
+            exact = product(special, dense).astype(np.float32)
+        assert np.array_equal(np.isnan(got), np.isnan(exact))
+        assert np.array_equal(np.isinf(got), np.isinf(exact))
+        assert np.array_equal(np.sign(got[np.isinf(got)]),
+                              np.sign(exact[np.isinf(exact)]))
+        # One term dominates this row: its own 2^-23 and the roundings (where
+        # its weight is zero the output is an ordinary sum, held to the bar).
+        np.testing.assert_allclose(
+            got[40], exact[40], rtol=4.0e-7,
+            atol=TOLERANCE * np.sqrt(256) * helpers.rms(dense))
+        error = helpers.normalized_error(got[others], exact[others], 256, 1.0,
+                                         helpers.rms(dense))
+        assert error <= TOLERANCE
