@@ -50,8 +50,6 @@ struct GemmShape {
     unsigned input_width;  // I: the weight's row length
 };
 
-constexpr unsigned kUnit = 32;  // contraction values per unit of a TilePlan
-
 // LDS beside the two tiles' buffers.
 template <bool kTall>
 struct GemmTables {
@@ -160,21 +158,22 @@ public:
         target_ = tile_address<kTall>(n, octet);
     }
     __device__ __forceinline__ void prime(unsigned) {}
-    __device__ __forceinline__ void load(unsigned k) {
-        word_ = __builtin_amdgcn_raw_buffer_load_b32(
+    __device__ __forceinline__ void load(unsigned k, int stage) {
+        word_[stage] = __builtin_amdgcn_raw_buffer_load_b32(
             codes_, inside_ ? flat_ / 2 : kOutside, k / 2, 0);
-        scale_ = scales_.load(flat_ + k, inside_);
+        scale_[stage] = scales_.load(flat_ + k, inside_);
     }
-    __device__ __forceinline__ void store(char* tile) {
+    template <bool kCareful>  // (a decoded weight is finite and is cut)
+    __device__ __forceinline__ void store(char* tile, int stage, float&) {
 #pragma clang fp contract(off)
-        const float scale = scales_.decode(scale_, tables_.factors);
+        const float scale = scales_.decode(scale_[stage], tables_.factors);
         float values[8];
-        decode_levels(word_, tables_.levels, values);
+        decode_levels(word_[stage], tables_.levels, values);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             values[i] = values[i] * scale;
         }
-        store_octet<false>(tile + target_, values);
+        store_octet<Split::Cut>(tile + target_, values);
     }
 
 private:
@@ -184,8 +183,8 @@ private:
     bool inside_;
     unsigned flat_;
     unsigned target_;
-    unsigned word_;
-    LoadedScale scale_;
+    unsigned word_[Tile<kTall>::kDepth];
+    LoadedScale scale_[Tile<kTall>::kDepth];
 };
 
 // value of lane (l ^ kXor), kXor in {1, 2, 4}, vector ALU only
@@ -257,39 +256,40 @@ public:
     }
     __device__ __forceinline__ void prime(unsigned k) {
         parity_ = 0;
-        load_scale(k);
-        store_scale();
+        load_scale(k, 0);
+        store_scale(0);
     }
-    __device__ __forceinline__ void load(unsigned k) {
-        word_ = __builtin_amdgcn_raw_buffer_load_b32(
+    __device__ __forceinline__ void load(unsigned k, int stage) {
+        word_[stage] = __builtin_amdgcn_raw_buffer_load_b32(
             codes_, lane_, k * (input_width_ / 2), 0);
-        load_scale(k + kStep);
+        load_scale(k + kStep, stage);
     }
-    __device__ __forceinline__ void store(char* tile) {
+    template <bool kCareful>  // (a decoded weight is finite and is cut)
+    __device__ __forceinline__ void store(char* tile, int stage, float&) {
 #pragma clang fp contract(off)
         const float* const scales =
             tables_.scales[parity_] + scale_source_;
         parity_ ^= 1U;
-        store_scale();
+        store_scale(stage);
         float values[8];
-        decode_levels(transpose_(word_), tables_.levels, values);
+        decode_levels(transpose_(word_[stage]), tables_.levels, values);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             values[i] = values[i] * scales[i];
         }
-        store_octet<false>(tile + target_, values);
+        store_octet<Split::Cut>(tile + target_, values);
     }
 
 private:
     static constexpr unsigned kStep = Tile<kTall>::kStep;
     static constexpr unsigned kScales = kTileN / 16 * kStep;
     // (past the last weight row: past the descriptors' extents)
-    __device__ __forceinline__ void load_scale(unsigned k) {
-        scale_ = scales_.load(scale_flat_ + k * input_width_, scale_inside_);
+    __device__ __forceinline__ void load_scale(unsigned k, int stage) {
+        scale_[stage] = scales_.load(scale_flat_ + k * input_width_, scale_inside_);
     }
-    __device__ __forceinline__ void store_scale() {
+    __device__ __forceinline__ void store_scale(int stage) {
         tables_.scales[parity_][threadIdx.x] =
-            scales_.decode(scale_, tables_.factors);
+            scales_.decode(scale_[stage], tables_.factors);
     }
     GemmTables<kTall>& tables_;
     ScaleReader<kDoubleQuantized> scales_;
@@ -302,8 +302,8 @@ private:
     bool scale_inside_;
     unsigned scale_flat_;
     unsigned parity_ = 0;
-    unsigned word_;
-    LoadedScale scale_;
+    unsigned word_[Tile<kTall>::kDepth];
+    LoadedScale scale_[Tile<kTall>::kDepth];
 };
 
 // The adapter's factors as a step's tiles: contraction value j of output row r
@@ -336,9 +336,10 @@ __device__ __forceinline__ void store_adapter_tiles(
                             ? source[(first + octet * 8 + i) * stride]
                             : 0.0F;
         }
-        store_octet<true>(tiles + (left ? 0U : Tile<kTall>::kLeftBytes) +
-                              tile_address<kTall>(place, octet),
-                          values);
+        store_octet<Split::Any>(tiles +
+                                    (left ? 0U : Tile<kTall>::kLeftBytes) +
+                                    tile_address<kTall>(place, octet),
+                                values);
     }
 }
 
@@ -383,7 +384,8 @@ __device__ __forceinline__ void gemm_segment(
             for (int slice = 0; slice < Tile<kTall>::kSlices; ++slice) {
                 if (16U * slice < count) {  // uniform
                     fragments.load(tiles, slice);
-                    fragments.multiply(sums, tiles, slice, [](int) {});
+                    fragments.template multiply<false>(sums, nullptr, 0,
+                                                       [](int) {});
                 }
             }
             __syncthreads();
@@ -391,15 +393,9 @@ __device__ __forceinline__ void gemm_segment(
         sums.fold(lora.scale);
     }
 
-    if (partial != nullptr) {  // uniform; layout [tile rows][kTileN]
-        for_each_output(sums, [&](unsigned row, unsigned column, float value) {
-            partial[row * kTileN + column] = value;
-        });
-        return;
-    }
     float addend[2] = {0.0F, 0.0F};
     if constexpr (!kBackward) {
-        if (bias != nullptr) {
+        if (bias != nullptr && partial == nullptr) {  // uniform
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const unsigned column = col0 + (threadIdx.x / 64 % 2) * 64 +
@@ -408,12 +404,13 @@ __device__ __forceinline__ void gemm_segment(
             }
         }
     }
-    for_each_output(sums, [&](unsigned row, unsigned column, float value) {
-        if (row0 + row < shape.rows && col0 + column < shape.columns) {
-            result[static_cast<std::size_t>(row0 + row) * shape.columns +
-                   col0 + column] = value + addend[column / 32 % 2];
-        }
-    });
+    store_outputs(sums,
+                  partial != nullptr
+                      ? partial  // layout [tile rows][kTileN]
+                      : result + static_cast<std::size_t>(row0) *
+                                     shape.columns + col0,
+                  partial != nullptr ? kTileN : shape.columns,
+                  shape.rows - row0, shape.columns - col0, addend);
 }
 
 template <bool kTall, bool kDoubleQuantized, bool kBackward>
@@ -474,9 +471,9 @@ void mfma_gemm_kernel(
 
 // Adds the parts of every unit-dealt tile that more than one workgroup worked
 // on, in ascending workgroup order, plus bias (the adapter term is in the
-// part that starts the contraction).  One thread
-// per output element: blockIdx.x is the tile among the unit-dealt ones,
-// blockIdx.y a run of 256 elements of it.
+// part that starts the contraction).  Four output elements per thread:
+// blockIdx.x is the tile among the unit-dealt ones, blockIdx.y a run of 1024
+// elements of it.
 template <unsigned kTileM>
 __global__ __launch_bounds__(256) void gemm_parts_kernel(
     const float* __restrict__ workspace, const float* __restrict__ bias,
@@ -490,24 +487,24 @@ __global__ __launch_bounds__(256) void gemm_parts_kernel(
         return;  // written directly by its only workgroup
     }
     const unsigned tile = plan.whole_tiles + dealt_tile;
-    const unsigned index = blockIdx.y * blockDim.x + threadIdx.x;
-    const unsigned m = index / kTileN;
-    const unsigned c = index % kTileN;
-    const unsigned row = plan.tile_row(tile) * kTileM + m;
-    const unsigned column = plan.tile_column(tile) * kTileN + c;
+    const unsigned index = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
+    const unsigned row = plan.tile_row(tile) * kTileM + index / kTileN;
+    const unsigned column = plan.tile_column(tile) * kTileN + index % kTileN;
     if (row >= shape.rows || column >= shape.columns) {
         return;
     }
-    const float* source = workspace + m * kTileN + c;
-    float sum = 0.0F;
-    for (unsigned group = first_group; group <= last_group; ++group) {
-        sum += source[static_cast<std::size_t>(plan.slot(group, dealt_tile)) *
-                      kTileM * kTileN];
-    }
+    floatx4 sum = add_parts<kTileM>(workspace, plan, dealt_tile, first_group,
+                                    last_group, index);
     if (bias != nullptr) {
-        sum += bias[column];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (column + e < shape.columns) {
+                sum[e] += bias[column + e];
+            }
+        }
     }
-    result[static_cast<std::size_t>(row) * shape.columns + column] = sum;
+    store_four(result + static_cast<std::size_t>(row) * shape.columns, column,
+               shape.columns, sum);
 }
 
 template <bool kTall, bool kDoubleQuantized, bool kBackward>
@@ -543,7 +540,7 @@ hipError_t launch_tiles(const LinearProblem& p, const GemmShape& shape,
         p.activations, p.weight, p.bias, p.result, workspace, shape, plan,
         p.block_shift, p.lora);
     if (groups != 0) {
-        const dim3 grid(tiles - plan.whole_tiles, kTileM * kTileN / 256);
+        const dim3 grid(tiles - plan.whole_tiles, kTileM * kTileN / 1024);
         gemm_parts_kernel<kTileM><<<grid, 256, 0, stream>>>(
             workspace, p.bias, p.result, shape, plan);
     }
@@ -579,17 +576,10 @@ unsigned tall_tile_columns(const GemmShape& shape) {
     return tall * 2 >= tiles_n ? tall : 0;
 }
 
-// Tall tiles decode and split the right operand once per 256 rows and are
-// faster per row (2048 rows of 11008 x 4096: 0.93 ms against 1.11; 4096 x 4096:
-// 334 against 402 us; 256 rows: 154 against 177 us), so the square ones are for
-// row counts that leave the last tall tile at most half full (128 rows: 107
-// against 133 us, 300 rows: 246 against 264 us).
 template <bool kDoubleQuantized, bool kBackward>
 hipError_t launch_encoding(const LinearProblem& p, const GemmShape& shape,
                            hipStream_t stream) {
-    constexpr unsigned kTallRows = Tile<true>::kTileM;
-    const unsigned last_rows = (shape.rows - 1) % kTallRows + 1;
-    return last_rows > kTallRows / 2
+    return use_tall_tiles(1, shape.rows, shape.contraction, shape.columns)
                ? launch_tiles<true, kDoubleQuantized, kBackward>(p, shape,
                                                                  stream)
                : launch_tiles<false, kDoubleQuantized, kBackward>(p, shape,

@@ -27,8 +27,8 @@
 // tile on an otherwise idle device takes 225 us of those 320 us.
 //
 // Infinities: hi + mid + lo of an infinite value would be a NaN, so it is
-// passed on as (0, 0, infinity): lo meets the other operand's hi alone, and
-// the sum is the infinity (or the NaN of infinity times zero) that fp32
+// passed on as (2^-126, 0, infinity): lo meets the other operand's hi alone,
+// and the sum is the infinity (or the NaN of infinity times zero) that fp32
 // arithmetic gives.  bf16 keeps fp32's exponent range and the matrix cores take
 // subnormal bf16 values as they are, so only values under 2^-110 have bits that
 // fall below bf16's smallest step, 2^-133, and are lost.
@@ -36,6 +36,7 @@
 
 #include "gemv_shared.hpp"
 #include "kernels.hpp"
+#include "tile_plan.hpp"
 
 #include <cstddef>
 #include <cstdint>
@@ -54,8 +55,22 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int kPlanes = 3;        // hi, mid, lo
 constexpr int kTileN = 128;       // output columns per workgroup
 constexpr unsigned kFragmentBytes = 1024;  // 32 rows x 16 contraction values
+constexpr unsigned kUnit = 32;  // contraction values per TilePlan unit
 constexpr unsigned kFlushValues = 256;  // contraction values per accumulation
 constexpr unsigned kOutside = 0xFFFFFFFFU;  // past every descriptor's extent
+
+// A pointer that is the same in every lane, in scalar registers: the compiler
+// takes quotients and 64-bit products to the vector unit and would read a
+// descriptor made from them lane by lane.
+__device__ __forceinline__ const float* uniform(const float* pointer) {
+    const std::uint64_t bits = reinterpret_cast<std::uint64_t>(pointer);
+    const unsigned low = __builtin_amdgcn_readfirstlane(
+        static_cast<unsigned>(bits));
+    const unsigned high = __builtin_amdgcn_readfirstlane(
+        static_cast<unsigned>(bits >> 32));
+    return reinterpret_cast<const float*>(
+        static_cast<std::uint64_t>(high) << 32 | low);
+}
 
 // Two values as three bf16 pairs (the first value in the low half).
 struct SplitPair {
@@ -105,17 +120,19 @@ __device__ __forceinline__ SplitPair split_pair(float a, float b) {
 // The same for any values.
 __device__ __forceinline__ SplitPair split_any_pair(float a, float b) {
     SplitPair out = split_pair<false>(a, b);
+    constexpr unsigned kSmallest = 0x0080U;  // bf16, normal
     if (__builtin_isinf(a)) {
-        out.hi &= 0xFFFF0000U;
+        const unsigned infinity = __builtin_bit_cast(unsigned, a) >> 16;
+        out.hi = (out.hi & 0xFFFF0000U) | (infinity & 0x8000U) | kSmallest;
         out.mid &= 0xFFFF0000U;
-        out.lo = (out.lo & 0xFFFF0000U) |
-                       (__builtin_bit_cast(unsigned, a) >> 16);
+        out.lo = (out.lo & 0xFFFF0000U) | infinity;
     }
     if (__builtin_isinf(b)) {
-        out.hi &= 0xFFFFU;
+        const unsigned infinity = __builtin_bit_cast(unsigned, b) >> 16;
+        out.hi =
+            (out.hi & 0xFFFFU) | ((infinity & 0x8000U) | kSmallest) << 16;
         out.mid &= 0xFFFFU;
-        out.lo = (out.lo & 0xFFFFU) |
-                       (__builtin_bit_cast(unsigned, b) & 0xFFFF0000U);
+        out.lo = (out.lo & 0xFFFFU) | infinity << 16;
     }
     return out;
 }
@@ -139,7 +156,8 @@ struct Tile {
     static constexpr int kStep = kTall ? 32 : 16;     // contraction per step
     static constexpr int kSlices = kStep / 16;  // matrix instructions' K
     static constexpr int kOctets = kStep / 8;   // a lane's eight values
-    static constexpr int kWorkgroupsPerUnit = kTall ? 1 : 2;
+    // steps whose operands are on their way into registers
+    static constexpr int kDepth = kTall ? 1 : 2;
     // workgroups the device holds at once
     static constexpr unsigned kPlaces = kTall ? 256 : 512;
     // rows of the left operand per pass of the workgroup (a float4 per thread)
@@ -153,6 +171,23 @@ struct Tile {
     // LDS of a workgroup: two buffers of both tiles
     static constexpr std::size_t kTileBytes = std::size_t{2} * kBufferBytes;
 };
+
+// Whether a product goes out in tall tiles: faster per row (2048 rows of 11008 x
+// 4096: 0.93 ms against 1.11; 4096 x 4096: 334 against 402 us; 256 rows: 154
+// against 177 us), unless they leave the last one at most half full (128 rows:
+// 107 against 133 us, 300 rows: 246 against 264 us) or there is less work than
+// 16 units for each compute unit: two square workgroups then cover each other's
+// starts and ends (2048 x 16 x 4096: 11 against 15 us, eight of 512 x 128 x
+// 512: 11 against 17 us).
+inline bool use_tall_tiles(std::size_t batch_count, std::size_t rows,
+                           std::size_t contraction, std::size_t columns) {
+    constexpr std::size_t kRows = Tile<true>::kTileM;
+    constexpr std::size_t kLeastUnits = 16 * Tile<true>::kPlaces;
+    const std::size_t tiles = batch_count * ((rows + kRows - 1) / kRows) *
+                              ((columns + kTileN - 1) / kTileN);
+    return (rows - 1) % kRows + 1 > kRows / 2 &&
+           tiles * ((contraction + kUnit - 1) / kUnit) >= kLeastUnits;
+}
 
 // Where the eight contraction values [8 * octet, 8 * octet + 8) of a row (or
 // column) of the tile lie in LDS, in bytes, plane 0.  The tile is kept as the
@@ -173,16 +208,19 @@ __device__ __forceinline__ unsigned tile_address(unsigned row,
 }
 
 // Splits eight values and writes them.
-template <bool kCareful>
+enum class Split { Cut, Rounded, Any };
+template <Split kSplit>
 __device__ __forceinline__ void store_octet(char* target,
                                             const float (&values)[8]) {
     uintx4 planes[kPlanes];
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
+        const float a = values[2 * p];
+        const float b = values[2 * p + 1];
         const SplitPair pair =
-            kCareful
-                ? split_any_pair(values[2 * p], values[2 * p + 1])
-                : split_pair<false>(values[2 * p], values[2 * p + 1]);
+            kSplit == Split::Any
+                ? split_any_pair(a, b)
+                : split_pair<kSplit == Split::Rounded>(a, b);
         planes[0][p] = pair.hi;
         planes[1][p] = pair.mid;
         planes[2][p] = pair.lo;
@@ -223,14 +261,14 @@ public:
     }
 
     // Requests pass `pass` of the step that starts at k.
-    __device__ __forceinline__ void load(unsigned k, int pass) {
+    __device__ __forceinline__ void load(unsigned k, int pass, int stage) {
         const unsigned step = k * static_cast<unsigned>(sizeof(float));
         if constexpr (kRagged) {
             // the row ends inside this step: value by value
             if (k + Tile<kTall>::kStep > width_) {  // uniform
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    values_[pass][e] = __builtin_bit_cast(
+                    values_[stage][pass][e] = __builtin_bit_cast(
                         float, __builtin_amdgcn_raw_buffer_load_b32(
                                    buffer_,
                                    k + column_ + e < width_
@@ -241,7 +279,7 @@ public:
                 return;
             }
         }
-        values_[pass] = __builtin_bit_cast(
+        values_[stage][pass] = __builtin_bit_cast(
             floatx4, __builtin_amdgcn_raw_buffer_load_b128(
                          buffer_, lane_[pass], step, 0));
     }
@@ -250,9 +288,9 @@ public:
     // `largest` is raised to the largest magnitude met, by which the caller
     // learns of values that may not be rounded.
     template <bool kCareful>
-    __device__ __forceinline__ void store(char* tile, int pass,
+    __device__ __forceinline__ void store(char* tile, int pass, int stage,
                                           float& largest) const {
-        const floatx4 v = values_[pass];
+        const floatx4 v = values_[stage][pass];
         SplitPair first;
         SplitPair second;
         if constexpr (kCareful) {
@@ -282,7 +320,7 @@ private:
     __amdgpu_buffer_rsrc_t buffer_;
     unsigned lane_[Tile<kTall>::kPasses];
     unsigned target_;
-    floatx4 values_[Tile<kTall>::kPasses];
+    floatx4 values_[Tile<kTall>::kDepth][Tile<kTall>::kPasses];
 };
 
 // Accumulators of a wavefront's 64 x 64 outputs.  Two levels: the matrix
@@ -350,12 +388,12 @@ public:
         load_left(tiles, slice, 0);
         load_right(tiles, slice, 0);
     }
-    // The slice's six products, 24 matrix instructions.  An operand plane is
-    // replaced by that of the next slice (`next_slice` of the buffer at
-    // `next`) as soon as its last product is issued, so that the next slice
+    // The slice's six products, 24 matrix instructions.  kRefill: an operand
+    // plane is replaced by that of the next slice (`next_slice` of the buffer
+    // at `next`) as soon as its last product is issued, so that the next slice
     // starts without waiting for LDS.  between(group) is called after each
     // group of four instructions; the replacements start after the third.
-    template <class Between>
+    template <bool kRefill, class Between>
     __device__ __forceinline__ void multiply(Accumulators& sums,
                                              const char* next, int next_slice,
                                              const Between& between) {
@@ -365,17 +403,25 @@ public:
         between(1);
         product(sums, 0, 1);
         between(2);
-        load_left(next, next_slice, 1);
-        load_right(next, next_slice, 1);
+        if constexpr (kRefill) {
+            load_left(next, next_slice, 1);
+            load_right(next, next_slice, 1);
+        }
         product(sums, 2, 0);
-        load_left(next, next_slice, 2);
+        if constexpr (kRefill) {
+            load_left(next, next_slice, 2);
+        }
         between(3);
         product(sums, 0, 2);
-        load_right(next, next_slice, 2);
+        if constexpr (kRefill) {
+            load_right(next, next_slice, 2);
+        }
         between(4);
         product(sums, 0, 0);
-        load_left(next, next_slice, 0);
-        load_right(next, next_slice, 0);
+        if constexpr (kRefill) {
+            load_left(next, next_slice, 0);
+            load_right(next, next_slice, 0);
+        }
         between(5);
     }
 
@@ -436,10 +482,10 @@ private:
 // one barrier stands in the middle of its last slice, whose operands are in
 // registers: behind it the other buffer is complete, this one may be
 // overwritten, and half a slice of matrix instructions covers the first reads
-// of the next step.  (The last step splits and writes what lies past the end,
-// which is never used; the descriptors' extents keep the loads inside the
-// operands.)  Returns the largest magnitude of the left operand that the
-// thread met (kCareful: zero).
+// of the next step.  (The step before the last requests what lies past the
+// end, which is never used; the descriptors' extents keep the loads inside the
+// operands.)  Returns the largest magnitude that the thread met and rounded
+// (kCareful: zero).
 template <bool kTall, bool kCareful, class Left, class Right>
 __device__ __forceinline__ float multiply_steps(Accumulators& sums, Left& left,
                                                 Right& right, char* tiles,
@@ -450,68 +496,93 @@ __device__ __forceinline__ float multiply_steps(Accumulators& sums, Left& left,
     constexpr int kSlices = Tile<kTall>::kSlices;
     constexpr unsigned kLeftBytes = Tile<kTall>::kLeftBytes;
     constexpr unsigned kBufferBytes = Tile<kTall>::kBufferBytes;
+    constexpr int kDepth = Tile<kTall>::kDepth;
     float largest = 0.0F;
-    const auto load_left = [&](unsigned k) {
+    const auto load_left = [&](unsigned k, int stage) {
 #pragma unroll
         for (int pass = 0; pass < kPasses; ++pass) {
-            left.load(k, pass);
+            left.load(k, pass, stage);
         }
     };
     right.prime(k_begin);
-    load_left(k_begin);
-    right.load(k_begin);
+#pragma unroll
+    for (int stage = 0; stage < kDepth; ++stage) {
+        load_left(k_begin + stage * kStep, stage);
+        right.load(k_begin + stage * kStep, stage);
+    }
     __syncthreads();  // nobody still reads the tiles of an earlier segment
 #pragma unroll
     for (int pass = 0; pass < kPasses; ++pass) {
-        left.template store<kCareful>(tiles, pass, largest);
+        left.template store<kCareful>(tiles, pass, 0, largest);
     }
-    right.store(tiles + kLeftBytes);
-    load_left(k_begin + kStep);
-    right.load(k_begin + kStep);
+    right.template store<kCareful>(tiles + kLeftBytes, 0, largest);
+    load_left(k_begin + kDepth * kStep, 0);
+    right.load(k_begin + kDepth * kStep, 0);
     __syncthreads();
 
     Fragments<kTall> fragments;
     fragments.load(tiles, 0);
     unsigned buffer = 0;
-    for (unsigned k0 = k_begin; k0 < k_end;) {
-        const unsigned fold_at = min(k0 + kFlushValues, k_end);
-        do {
-            const char* const current = tiles + buffer * kBufferBytes;
-            char* const target = tiles + (buffer ^ 1U) * kBufferBytes;
-            if constexpr (kSlices == 2) {
-                fragments.multiply(sums, current, 1, [&](int group) {
-                    if (group == 0) {
-                        right.store(target + kLeftBytes);
-                        right.load(k0 + 2 * kStep);
-                    } else if (group <= kPasses) {
-                        left.template store<kCareful>(target, group - 1,
-                                                      largest);
-                    } else {
-                        load_left(k0 + 2 * kStep);
-                    }
-                });
+    unsigned k0 = k_begin;
+    // One step; the next one's operands are in registers `stage`.
+    const auto advance = [&](int stage) {
+        const char* const current = tiles + buffer * kBufferBytes;
+        char* const target = tiles + (buffer ^ 1U) * kBufferBytes;
+        const unsigned k_load = k0 + (kDepth + 1) * kStep;
+        // after group `group` of the slice that precedes the barrier, or (tall)
+        // of the slice before that
+        const auto refill = [&](int group) {
+            if (group == 0) {
+                right.template store<kCareful>(target + kLeftBytes, stage,
+                                               largest);
+                right.load(k_load, stage);
+            } else if (group <= kPasses) {
+                left.template store<kCareful>(target, group - 1, stage,
+                                              largest);
             }
-            fragments.multiply(sums, target, 0, [&](int group) {
-                if constexpr (kSlices == 1) {
-                    if (group == 0) {
-                        right.store(target + kLeftBytes);
-                        right.load(k0 + 2 * kStep);
-                    } else if (group <= kPasses) {
-                        left.template store<kCareful>(target, group - 1,
-                                                      largest);
-                    } else if (group == 3) {
-                        load_left(k0 + 2 * kStep);
-                    }
-                }
-                if (group == 2) {
-                    __syncthreads();
-                }
-            });
-            buffer ^= 1U;
-            k0 += kStep;
+            if (group == (kSlices == 2 ? 5 : kPasses)) {
+                load_left(k_load, stage);
+            }
+        };
+        if constexpr (kSlices == 2) {
+            fragments.template multiply<true>(sums, current, 1, refill);
+        }
+        fragments.template multiply<true>(sums, target, 0, [&](int group) {
+            if constexpr (kSlices == 1) {
+                refill(group);
+            }
+            if (group == 2) {
+                __syncthreads();
+            }
+        });
+        buffer ^= 1U;
+        k0 += kStep;
+    };
+    // Rounds of kDepth steps (a unit holds one or two whole rounds); the last
+    // one ends with a step that has nothing to refill.
+    constexpr unsigned kRound = kDepth * kStep;
+    static_assert(kUnit % kRound == 0);
+    while (k0 + kRound < k_end) {
+        const unsigned fold_at = min(k0 + kFlushValues, k_end - kRound);
+        do {
+#pragma unroll
+            for (int step = 1; step <= kDepth; ++step) {
+                advance(step % kDepth);
+            }
         } while (k0 < fold_at);
         sums.fold();
     }
+#pragma unroll
+    for (int step = 1; step < kDepth; ++step) {
+        advance(step % kDepth);
+    }
+    const auto nothing = [](int) {};
+    if constexpr (kSlices == 2) {
+        fragments.template multiply<true>(sums, tiles + buffer * kBufferBytes,
+                                          1, nothing);
+    }
+    fragments.template multiply<false>(sums, nullptr, 0, nothing);
+    sums.fold();
     __syncthreads();  // the tiles have been read
     return largest;
 }
@@ -532,25 +603,98 @@ __device__ __forceinline__ void multiply_tile(Accumulators& sums, Left& left,
     }
 }
 
-// Calls store(row in tile, column in tile, value) for every output of the
-// lane.  Accumulator element e of lane l is output row 8 * (e / 4) +
-// 4 * (l / 32) + e % 4, column l % 32 of its 32 x 32 block.
-template <class Store>
-__device__ __forceinline__ void for_each_output(const Accumulators& sums,
-                                                const Store& store) {
+// Writes a wavefront's 64 x 64 outputs, plus addend[j] in the columns of its
+// block column j, to `target` (row 0, column 0 of the tile; `stride` floats per
+// row, below 2^24), those in the first `rows` rows and `columns` columns of the
+// tile.  Buffer stores: what lies outside is past the descriptor's extent or
+// carries an offset that is, and nothing branches.  Accumulator element e of
+// lane l is output row 8 * (e / 4) + 4 * (l / 32) + e % 4, column l % 32 of its
+// 32 x 32 block.
+__device__ __forceinline__ void store_outputs(const Accumulators& sums,
+                                              float* target, unsigned stride,
+                                              unsigned rows, unsigned columns,
+                                              const float (&addend)[2]) {
     const unsigned lane = threadIdx.x % 64;
-    const unsigned wave = threadIdx.x / 64;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const unsigned first_row = wave / 2 * 64;
+    const unsigned wave_rows =
+        first_row < rows ? min(rows - first_row, 64U) : 0U;
+    const unsigned row_bytes = stride * static_cast<unsigned>(sizeof(float));
+    const __amdgpu_buffer_rsrc_t buffer = make_buffer(
+        uniform(target + static_cast<std::size_t>(first_row) * stride),
+        __builtin_amdgcn_readfirstlane(wave_rows * row_bytes));
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int j = 0; j < 2; ++j) {
+        const unsigned column = wave % 2 * 64 + j * 32 + lane % 32;
+        const unsigned offset =
+            column < columns
+                ? lane / 32 * 4 * row_bytes +
+                      column * static_cast<unsigned>(sizeof(float))
+                : kOutside;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const unsigned column = (wave % 2) * 64 + j * 32 + lane % 32;
+        for (int i = 0; i < 2; ++i) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                const unsigned row = (wave / 2) * 64 + i * 32 + 8 * (e / 4) +
-                                     4 * (lane / 32) + e % 4;
-                store(row, column, sums.total[i][j][e]);
+                __builtin_amdgcn_raw_buffer_store_b32(
+                    __builtin_bit_cast(unsigned,
+                                       sums.total[i][j][e] + addend[j]),
+                    buffer, offset,
+                    __builtin_amdgcn_readfirstlane(
+                        (i * 32 + 8 * (e / 4) + e % 4) * row_bytes),
+                    0);
             }
+        }
+    }
+}
+
+// The sum of the parts of a unit-dealt tile, in ascending workgroup order, for
+// the four neighbouring outputs from `index` ([tile rows][kTileN]) on.  Four
+// parts at a time are requested before the first is added (one after the other,
+// sixteen parts are sixteen trips to memory: 128 rows of 4096 x 11008 spent
+// 11 of 88 us here, now 7).
+template <unsigned kTileM>
+__device__ __forceinline__ floatx4 add_parts(const float* workspace,
+                                             const TilePlan& plan,
+                                             unsigned dealt_tile,
+                                             unsigned first_group,
+                                             unsigned last_group,
+                                             unsigned index) {
+    constexpr std::size_t kSlot = std::size_t{kTileM} * kTileN;
+    const auto part = [&](unsigned slot) {
+        return *reinterpret_cast<const floatx4*>(workspace + slot * kSlot +
+                                                 index);
+    };
+    // (every workgroup but the first starts inside this tile)
+    floatx4 sum = part(plan.slot(first_group, dealt_tile));
+    unsigned group = first_group + 1;
+    for (; group + 3 <= last_group; group += 4) {
+        floatx4 parts[4];
+#pragma unroll
+        for (unsigned p = 0; p < 4; ++p) {
+            parts[p] = part(2 * (group + p));
+        }
+#pragma unroll
+        for (unsigned p = 0; p < 4; ++p) {
+            sum += parts[p];
+        }
+    }
+    for (; group <= last_group; ++group) {
+        sum += part(2 * group);
+    }
+    return sum;
+}
+
+// Writes four neighbouring outputs of a row of `columns`, from `column` on.
+__device__ __forceinline__ void store_four(float* row, unsigned column,
+                                           unsigned columns, floatx4 values) {
+    if (columns % 4 == 0 && reinterpret_cast<std::uintptr_t>(row) % 16 == 0) {
+        *reinterpret_cast<floatx4*>(row + column) = values;
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (column + e < columns) {
+            row[column + e] = values[e];
         }
     }
 }

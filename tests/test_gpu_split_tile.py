@@ -100,3 +100,53 @@ def test_infinite_and_huge_values(gpu, package, oracle, rows):
         error = helpers.normalized_error(got[others], exact[others], 256, 1.0,
                                          helpers.rms(dense))
         assert error <= TOLERANCE
+
+
+@pytest.mark.parametrize("batch,rows,shared,columns", [
+    (1, 33, 1, 64),           # one contraction value
+    (1, 129, 31, 127),        # rows that start at any alignment
+    (3, 50, 33, 130),         # one value past a unit; batches back to back
+    (2, 256, 257, 129),       # 256-row tiles, one fold and one value
+    (1, 257, 1023, 1025),     # dealt in runs, every edge ragged
+    (5, 131, 515, 517),       # runs that cross from one matrix to the next
+])
+def test_dense_matmul_edges(gpu, batch, rows, shared, columns):
+    import torch
+    left = helpers.normal(906, (batch, rows, shared), 1.0)
+    right = helpers.normal(907, (batch, shared, columns), 0.05)
+    got = gpu.matmul(torch.from_numpy(left).cuda(),
+                     torch.from_numpy(right).cuda()).cpu().numpy()
+    exact = left.astype(np.float64) @ right.astype(np.float64)
+    error = np.abs(got - exact).max() / (0.05 * np.sqrt(shared))
+    assert error <= TOLERANCE, f"{error:.3g}"
+
+
+def test_dense_matmul_of_infinite_values(gpu):
+    """Infinities on either side, and on both sides of one product."""
+    import torch
+    left = helpers.normal(908, (1, 140, 70), 1.0)
+    right = helpers.normal(909, (1, 70, 150), 1.0)
+    left[0, 4, 10] = np.inf
+    left[0, 9, 20] = -np.inf
+    right[0, 20, 30] = np.inf       # meets the -inf of row 9
+    # A value that rounds to infinity in bf16.  Its products stay below
+    # 0.5 x 3.4e38 (|N(0, 1)| < 5): sums in 64 bits do not overflow where fp32
+    # would, and infinity less an overflow is not a number.
+    right[0, 33, 40] = np.float32(-3.4e38)
+    left[0, :, 33] *= np.float32(0.1)
+    right[0, 60, 50] = np.nan
+    got = gpu.matmul(torch.from_numpy(left).cuda(),
+                     torch.from_numpy(right).cuda()).cpu().numpy()
+    with np.errstate(invalid="ignore", over="ignore"):
+        exact = (left.astype(np.float64) @
+                 right.astype(np.float64)).astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(exact))
+    infinite = np.isinf(exact)
+    assert np.array_equal(np.isinf(got), infinite)
+    assert np.array_equal(got[infinite], exact[infinite])
+    # one term dominates this column: its own 2^-23 and the roundings
+    huge = np.isfinite(exact[0, :, 40]) & (np.abs(exact[0, :, 40]) > 1.0e30)
+    np.testing.assert_allclose(got[0, huge, 40], exact[0, huge, 40],
+                               rtol=4.0e-7)
+    plain = np.isfinite(exact) & (np.abs(exact) < 1.0e3)
+    assert np.abs(got - exact)[plain].max() <= TOLERANCE * np.sqrt(70)
