@@ -190,8 +190,8 @@ hipError_t launch_dense_matmul(const float* left, const float* right,
 // nf4_quantize.hip -- the quantizer.  fp32_scales always receives the block
 // scales; scale_codes == nullptr means plain fp32 scales, otherwise the
 // scales are double-quantised into scale_codes / second_level / *offset.
-// status is a device word the kernels OR error bits into (1: non-finite
-// source value, 2: the scale mean is not finite).
+// status is a device word that receives error bits (1: non-finite source
+// value, 2: the scale mean is not finite).
 struct QuantizeProblem {
     const float* values;
     std::size_t element_count;
@@ -202,7 +202,8 @@ struct QuantizeProblem {
     float* second_level;
     unsigned second_level_shift;
     float* offset;     // device
-    unsigned* status;  // device, zeroed by the caller
+    unsigned* status;  // device
+    void* workspace;   // device, kStreamWorkspaceBytes
 };
 void launch_quantize(const QuantizeProblem& problem, hipStream_t stream);
 

@@ -30,7 +30,7 @@ struct Nf4WeightView {
     float offset;
 };
 
-__device__ __constant__ const float kNf4Codebook[16] = {
+__device__ __constant__ constexpr float kNf4Codebook[16] = {
     -1.0F,
     -0.6961928009986877F,
     -0.5250730514526367F,

@@ -16,16 +16,27 @@
 //                 every operation rounded on its own
 //
 // The one step whose result depends on evaluation order is the double sum.
-// It is evaluated in parallel only when that provably cannot matter: the
-// scales are non-negative fp32 values, so if count * max < 2^53 * (smallest
-// unit in the last place among the non-zero scales), every partial sum in
-// every order is exactly representable and all orders give the same double.
-// Otherwise one thread adds the scales in index order, as the reference does.
+// It is evaluated in parallel only where that provably cannot matter: the
+// scales are non-negative fp32 values, all of them multiples of u, the
+// smallest unit in the last place among the non-zero ones, so every partial
+// sum below 2^53 u is exact in double.  A sum that comes out below 2^53 u had
+// no partial sum that reached it (sums of non-negative values do not shrink,
+// and 2^53 u itself is representable), so every order gives it.  Otherwise one
+// thread adds the scales in index order, as the reference does.
+//
+// What bounds it: memory; the weight is read once, its scales stay in
+// registers between the maximum and the codes, and the sum of the scales is
+// taken on the way.  11008 x 4096, block 64, nested: 37 us for the pass over
+// the weight (5.5 TB/s) and 9 us for the scales, 79 us for the whole call with
+// its wait.  A pass for the scales (70 us), one for the codes by sixteen
+// distances each (94 us) and one workgroup for the mean (229 us) took 435 us.
 
 #include "kernels.hpp"
 #include "nf4_decode.hpp"
 
+#include <bit>
 #include <cfloat>
+#include <climits>
 
 namespace rthip {
 namespace {
@@ -33,185 +44,306 @@ namespace {
 // Bits of the status word the kernels report through.
 constexpr unsigned kNonFiniteSource = 1U;
 constexpr unsigned kOffsetOverflow = 2U;
+constexpr unsigned kInfinityBits = 0x7F800000U;
 
-__device__ __forceinline__ unsigned nearest_code(float normalized) {
-    unsigned best_code = 0;
-    float best_distance = fabsf(normalized - kNf4Codebook[0]);
-#pragma unroll
-    for (unsigned code = 1; code < 16; ++code) {
-        const float distance = fabsf(normalized - kNf4Codebook[code]);
-        if (distance < best_distance) {
-            best_distance = distance;
-            best_code = code;
+// The linear scan's result only grows with the normalised value: between two
+// neighbouring entries the rounded distance to the lower one does not shrink
+// and that to the upper one does not grow.  kThresholds[i] is the smallest
+// value at which the scan prefers entry i + 1 to entry i.
+struct Thresholds {
+    float at[15];
+};
+consteval Thresholds find_thresholds() {
+    // floats in ascending order as integers, and back
+    const auto order = [](float value) {
+        const int bits = std::bit_cast<int>(value);
+        return bits < 0 ? INT_MIN - bits : bits;
+    };
+    const auto value_of = [](int place) {
+        return std::bit_cast<float>(place < 0 ? INT_MIN - place : place);
+    };
+    Thresholds out{};
+    for (int i = 0; i < 15; ++i) {
+        const float lower = kNf4Codebook[i];
+        const float upper = kNf4Codebook[i + 1];
+        int below = order(lower);  // prefers i
+        int above = order(upper);  // prefers i + 1
+        while (above - below > 1) {
+            const int middle = below + (above - below) / 2;
+            const float value = value_of(middle);
+            if (upper - value < value - lower) {
+                above = middle;
+            } else {
+                below = middle;
+            }
         }
+        out.at[i] = value_of(above);
     }
-    return best_code;
+    return out;
+}
+constexpr Thresholds kThresholds = find_thresholds();
+
+// [-1, 1] in 31 intervals, narrower than the distance between two thresholds
+// (0.0646 against 0.0804): the codes of an interval are those from `code` on,
+// one more from `threshold` on.  One LDS read (32 entries in 64 banks: no
+// conflicts) and one comparison in place of sixteen distances.
+struct Interval {
+    float threshold;
+    unsigned code;
+};
+constexpr int kIntervals = 32;  // the first is for values that are no numbers
+__device__ __forceinline__ unsigned interval_of(float normalized) {
+    // 1..31 in the low bits: the sum's unit in the last place is one
+    return __float_as_uint(
+               __builtin_fmaf(normalized, 15.49F, 0x1p23F + 16.0F)) %
+           kIntervals;
+}
+__device__ __forceinline__ Interval make_interval(unsigned interval) {
+    Interval out{INFINITY, 0};
+#pragma unroll
+    for (int i = 0; i < 15; ++i) {
+        const unsigned place = interval_of(kThresholds.at[i]);
+        out.code += place < interval ? 1U : 0U;
+        out.threshold = place == interval ? kThresholds.at[i] : out.threshold;
+    }
+    return out;
 }
 
-// One wavefront per quantisation block: scale = max |w|.
-__global__ __launch_bounds__(256) void block_scale_kernel(
+// What a workgroup of pack_kernel found: the sum of its scales, the biased
+// exponent of the smallest non-zero one (INT_MAX: none), status bits.
+struct ScaleRecord {
+    double sum;
+    int least_exponent;
+    unsigned status;
+};
+__device__ __forceinline__ ScaleRecord combine(const ScaleRecord& a,
+                                               const ScaleRecord& b) {
+    return {a.sum + b.sum, min(a.least_exponent, b.least_exponent),
+            a.status | b.status};
+}
+
+constexpr int kPackThreads = 512;
+constexpr std::size_t kPackValues = kPackThreads * 8;
+// Enough for every workgroup the device holds at once.
+constexpr unsigned kMaxRecords = 1024;
+static_assert(kMaxRecords * sizeof(ScaleRecord) <= kStreamWorkspaceBytes);
+
+// A thread takes eight consecutive weights, a workgroup 4096 at a time; the
+// threads of a quantisation block (4 to 512 neighbours) exchange their largest
+// magnitude.  kWide: a block spans wavefronts (block sizes from 1024 on).
+// records null: fp32 scales, status bits go to *status.
+template <bool kWide>
+__global__ __launch_bounds__(kPackThreads) void pack_kernel(
     const float* __restrict__ values, std::size_t element_count,
-    unsigned block_shift, std::size_t block_count, float* __restrict__ scales,
+    unsigned block_shift, bool aligned, float* __restrict__ scales,
+    std::uint8_t* __restrict__ codes, ScaleRecord* __restrict__ records,
     unsigned* __restrict__ status
 ) {
-    const std::size_t waves_per_grid =
-        static_cast<std::size_t>(gridDim.x) * (blockDim.x / 64);
-    const unsigned lane = threadIdx.x % 64;
-    const std::size_t block_size = std::size_t{1} << block_shift;
-    bool bad = false;
-    for (std::size_t block =
-             static_cast<std::size_t>(blockIdx.x) * (blockDim.x / 64) +
-             threadIdx.x / 64;
-         block < block_count; block += waves_per_grid) {
-        const std::size_t begin = block << block_shift;
-        const std::size_t end = begin + block_size < element_count
-                                    ? begin + block_size
-                                    : element_count;
-        float scale = 0.0F;
-        for (std::size_t index = begin + lane; index < end; index += 64) {
-            const float value = values[index];
-            bad = bad || !isfinite(value);
-            const float magnitude = fabsf(value);
-            scale = scale < magnitude ? magnitude : scale;
-        }
-#pragma unroll
-        for (int offset = 32; offset >= 1; offset /= 2) {
-            const float other = __shfl_xor(scale, offset, 64);
-            scale = scale < other ? other : scale;
-        }
-        if (lane == 0) {
-            scales[block] = scale;
-        }
+    constexpr unsigned kWaves = kPackThreads / 64;
+    __shared__ Interval intervals[kIntervals];
+    __shared__ unsigned wave_largest[2][kWaves];
+    __shared__ ScaleRecord wave_records[kWaves];
+    if (threadIdx.x < kIntervals) {
+        intervals[threadIdx.x] = make_interval(threadIdx.x);
     }
-    if (bad) {
-        atomicOr(status, kNonFiniteSource);
-    }
-}
+    __syncthreads();
 
-// One thread per eight consecutive weights (four code bytes); eight weights
-// never straddle a block because block sizes are multiples of 32.
-__global__ __launch_bounds__(256) void encode_kernel(
-    const float* __restrict__ values, std::size_t element_count,
-    unsigned block_shift, const float* __restrict__ scales,
-    std::uint8_t* __restrict__ codes
-) {
-    const std::size_t group_count = (element_count + 7) / 8;
-    const std::size_t stride =
-        static_cast<std::size_t>(gridDim.x) * blockDim.x;
-    for (std::size_t group =
-             static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-         group < group_count; group += stride) {
-        const std::size_t first = group * 8;
-        const float scale = scales[first >> block_shift];
+    const unsigned wave = threadIdx.x / 64;
+    const unsigned block_threads = 1U << (block_shift - 3);
+    const unsigned block_lanes = min(block_threads, 64U);
+    const std::size_t byte_count = (element_count + 1) / 2;
+    ScaleRecord record{0.0, INT_MAX, 0U};
+    unsigned turn = 0;
+    for (std::size_t tile = blockIdx.x; tile * kPackValues < element_count;
+         tile += gridDim.x) {
+        const std::size_t first = tile * kPackValues + threadIdx.x * 8;
+        float value[8];
+        if (aligned && first + 8 <= element_count) {
+            const float4 low =
+                *reinterpret_cast<const float4*>(values + first);
+            const float4 high =
+                *reinterpret_cast<const float4*>(values + first + 4);
+            value[0] = low.x;
+            value[1] = low.y;
+            value[2] = low.z;
+            value[3] = low.w;
+            value[4] = high.x;
+            value[5] = high.y;
+            value[6] = high.z;
+            value[7] = high.w;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                value[i] =
+                    first + i < element_count ? values[first + i] : 0.0F;
+            }
+        }
+        // magnitudes compare like their bits; above infinity: not a number
+        unsigned largest = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            largest = max(largest, __float_as_uint(value[i]) & 0x7FFFFFFFU);
+        }
+        for (unsigned step = 1; step < block_lanes; step *= 2) {
+            largest = max(largest, static_cast<unsigned>(__shfl_xor(
+                                       static_cast<int>(largest),
+                                       static_cast<int>(step), 64)));
+        }
+        if constexpr (kWide) {
+            // (two arrays in turn: one barrier a tile)
+            if (threadIdx.x % 64 == 0) {
+                wave_largest[turn][wave] = largest;
+            }
+            __syncthreads();
+            const unsigned block_waves = block_threads / 64;
+            const unsigned first_wave = wave / block_waves * block_waves;
+            for (unsigned other = 0; other < block_waves; ++other) {
+                largest =
+                    max(largest, wave_largest[turn][first_wave + other]);
+            }
+            turn ^= 1U;
+        }
+        const float scale = __uint_as_float(largest);
+        if (largest >= kInfinityBits) {
+            record.status = kNonFiniteSource;
+        }
+        if (first >= element_count) {
+            continue;  // (kWide: the tile is the last one, see the loop)
+        }
+        if (threadIdx.x % block_threads == 0) {
+            scales[first >> block_shift] = scale;
+            record.sum += static_cast<double>(scale);
+            if (largest != 0) {
+                record.least_exponent =
+                    min(record.least_exponent,
+                        max(static_cast<int>(largest >> 23), 1));
+            }
+        }
         unsigned packed = 0;
 #pragma unroll
-        for (unsigned i = 0; i < 8; ++i) {
-            const std::size_t index = first + i;
-            unsigned code = 0;  // an unused nibble stays zero
-            if (index < element_count) {
-                code = scale == 0.0F ? 7U : nearest_code(values[index] / scale);
-            }
+        for (int i = 0; i < 8; ++i) {
+            const float normalized = value[i] / scale;
+            const Interval interval = intervals[interval_of(normalized)];
+            const unsigned code =
+                interval.code + (normalized >= interval.threshold ? 1U : 0U);
             packed |= code << (4 * i);
         }
-        const std::size_t byte_count = (element_count + 1) / 2;
-        const std::size_t first_byte = group * 4;
-        if (first_byte + 4 <= byte_count) {
+        if (largest == 0) {
+            packed = 0x77777777U;
+        }
+        const std::size_t first_byte = first / 2;
+        if (first + 8 <= element_count) {
             // four-byte groups start at multiples of four bytes
             *reinterpret_cast<unsigned*>(codes + first_byte) = packed;
         } else {
+            // an unused nibble stays zero
+            packed &= (1U << (4 * (element_count - first))) - 1U;
             for (unsigned i = 0; first_byte + i < byte_count; ++i) {
                 codes[first_byte + i] =
                     static_cast<std::uint8_t>((packed >> (8 * i)) & 0xFFU);
             }
         }
     }
+    if (records == nullptr) {
+        if (record.status != 0) {
+            atomicOr(status, record.status);
+        }
+        return;
+    }
+#pragma unroll
+    for (int step = 32; step >= 1; step /= 2) {
+        record = combine(
+            record,
+            {__shfl_xor(record.sum, step, 64),
+             __shfl_xor(record.least_exponent, step, 64),
+             static_cast<unsigned>(__shfl_xor(
+                 static_cast<int>(record.status), step, 64))});
+    }
+    if (threadIdx.x % 64 == 0) {
+        wave_records[wave] = record;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (unsigned other = 1; other < kWaves; ++other) {
+            record = combine(record, wave_records[other]);
+        }
+        records[blockIdx.x] = record;
+    }
 }
 
-// offset = (float)(sum of the scales in double / count), by ONE workgroup.
-constexpr int kMeanThreads = 1024;
+// The scales' mean, then their codes; one wavefront per group of
+// second-level-block scales.  Every workgroup adds the records for itself, in
+// the same order (at most 16 KB from L2, where a launch of one workgroup
+// between the two kernels took longer); the first one reports the mean and the
+// status.
+constexpr int kEncodeThreads = 256;
 
-__global__ __launch_bounds__(kMeanThreads) void scale_mean_kernel(
-    const float* __restrict__ scales, std::size_t count,
-    float* __restrict__ offset_out, unsigned* __restrict__ status
+__global__ __launch_bounds__(kEncodeThreads) void scale_encode_kernel(
+    const float* __restrict__ scales, std::size_t count, unsigned group_shift,
+    std::size_t group_count, const ScaleRecord* __restrict__ records,
+    unsigned record_count, float* __restrict__ offset_out,
+    unsigned* __restrict__ status, std::uint8_t* __restrict__ scale_codes,
+    float* __restrict__ second_level
 ) {
-    __shared__ double sums[kMeanThreads];
-    __shared__ int largest_exponent[kMeanThreads];
-    __shared__ int smallest_ulp[kMeanThreads];
-
-    // exponent of a value's unit in the last place; INT_MAX for zero
-    double sum = 0.0;
-    int top = INT_MIN;
-    int ulp = INT_MAX;
-    for (std::size_t index = threadIdx.x; index < count;
-         index += kMeanThreads) {
-        const float value = scales[index];
-        sum += static_cast<double>(value);
-        if (value != 0.0F) {
-            const unsigned bits = __float_as_uint(value);
-            const int biased = static_cast<int>((bits >> 23) & 0xFFU);
-            const int exponent = (biased == 0 ? 1 : biased) - 127;
-            top = max(top, exponent);
-            ulp = min(ulp, exponent - 23);
-        }
+#pragma clang fp contract(off)
+    __shared__ ScaleRecord sums[kEncodeThreads];
+    constexpr unsigned kStaged = 1024;
+    __shared__ float staged[kStaged];
+    ScaleRecord record{0.0, INT_MAX, 0U};
+    for (unsigned index = threadIdx.x; index < record_count;
+         index += kEncodeThreads) {
+        record = combine(record, records[index]);
     }
-    sums[threadIdx.x] = sum;
-    largest_exponent[threadIdx.x] = top;
-    smallest_ulp[threadIdx.x] = ulp;
+    sums[threadIdx.x] = record;
     __syncthreads();
-    for (int width = kMeanThreads / 2; width >= 1; width /= 2) {
-        if (static_cast<int>(threadIdx.x) < width) {
-            sums[threadIdx.x] += sums[threadIdx.x + width];
-            largest_exponent[threadIdx.x] =
-                max(largest_exponent[threadIdx.x],
-                    largest_exponent[threadIdx.x + width]);
-            smallest_ulp[threadIdx.x] = min(smallest_ulp[threadIdx.x],
-                                            smallest_ulp[threadIdx.x + width]);
+    for (unsigned width = kEncodeThreads / 2; width >= 1; width /= 2) {
+        if (threadIdx.x < width) {
+            sums[threadIdx.x] =
+                combine(sums[threadIdx.x], sums[threadIdx.x + width]);
         }
         __syncthreads();
     }
-    if (threadIdx.x != 0) {
-        return;
-    }
-    double total = sums[0];
-    if (largest_exponent[0] != INT_MIN) {
-        // every value < 2^(top + 1), so any partial sum < count * 2^(top + 1)
-        // <= 2^(count_bits + top + 1); exact in double while that stays
-        // <= 2^53 * 2^ulp.
-        int count_bits = 0;
-        while ((std::size_t{1} << count_bits) < count) {
-            ++count_bits;
-        }
-        const bool order_free =
-            count_bits + largest_exponent[0] + 1 <= 53 + smallest_ulp[0];
-        if (!order_free) {
-            total = 0.0;
-            for (std::size_t index = 0; index < count; ++index) {
-                total += static_cast<double>(scales[index]);
+    record = sums[0];
+    // 2^53 units in the last place of the smallest scale: the exponent of
+    // that unit is least_exponent - 127 - 23
+    const bool order_free =
+        record.status != 0 || record.least_exponent == INT_MAX ||
+        record.sum < ldexp(1.0, 53 - 127 - 23 + record.least_exponent);
+    if (!order_free) {  // uniform
+        double total = 0.0;
+        for (std::size_t first = 0; first < count; first += kStaged) {
+            __syncthreads();
+            for (unsigned i = threadIdx.x; i < kStaged; i += kEncodeThreads) {
+                staged[i] = first + i < count ? scales[first + i] : 0.0F;
+            }
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                // (zeros past the end change no sum)
+#pragma unroll 16
+                for (unsigned i = 0; i < kStaged; ++i) {
+                    total += static_cast<double>(staged[i]);
+                }
             }
         }
+        if (threadIdx.x == 0) {
+            sums[0].sum = total;
+        }
+        __syncthreads();
+        record.sum = sums[0].sum;
     }
     const float offset =
-        static_cast<float>(total / static_cast<double>(count));
-    *offset_out = offset;
-    if (!isfinite(offset)) {
-        atomicOr(status, kOffsetOverflow);
+        static_cast<float>(record.sum / static_cast<double>(count));
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *offset_out = offset;
+        *status = record.status | (isfinite(offset) ? 0U : kOffsetOverflow);
     }
-}
 
-// One wavefront per group of second-level-block scales.
-__global__ __launch_bounds__(256) void scale_encode_kernel(
-    const float* __restrict__ scales, std::size_t count, unsigned group_shift,
-    std::size_t group_count, const float* __restrict__ offset_pointer,
-    std::uint8_t* __restrict__ scale_codes, float* __restrict__ second_level
-) {
-#pragma clang fp contract(off)
-    const float offset = *offset_pointer;
     const std::size_t waves_per_grid =
-        static_cast<std::size_t>(gridDim.x) * (blockDim.x / 64);
+        static_cast<std::size_t>(gridDim.x) * (kEncodeThreads / 64);
     const unsigned lane = threadIdx.x % 64;
     const std::size_t group_size = std::size_t{1} << group_shift;
     for (std::size_t group =
-             static_cast<std::size_t>(blockIdx.x) * (blockDim.x / 64) +
+             static_cast<std::size_t>(blockIdx.x) * (kEncodeThreads / 64) +
              threadIdx.x / 64;
          group < group_count; group += waves_per_grid) {
         const std::size_t begin = group << group_shift;
@@ -247,38 +379,43 @@ __global__ __launch_bounds__(256) void scale_encode_kernel(
     }
 }
 
-unsigned grid_for(std::size_t items, std::size_t per_block) {
-    constexpr std::size_t kMaxBlocks = 256 * 32;
-    std::size_t blocks = (items + per_block - 1) / per_block;
-    if (blocks == 0) {
-        blocks = 1;
-    }
-    return static_cast<unsigned>(blocks < kMaxBlocks ? blocks : kMaxBlocks);
+unsigned grid_for(std::size_t items, std::size_t per_block, unsigned most) {
+    const std::size_t blocks = (items + per_block - 1) / per_block;
+    return static_cast<unsigned>(blocks < most ? blocks : most);
 }
 
 }  // namespace
 
 void launch_quantize(const QuantizeProblem& p, hipStream_t stream) {
+    const bool nested = p.scale_codes != nullptr;
     const std::size_t block_count =
         (p.element_count + (std::size_t{1} << p.block_shift) - 1) >>
         p.block_shift;
-    block_scale_kernel<<<grid_for(block_count, 4), 256, 0, stream>>>(
-        p.values, p.element_count, p.block_shift, block_count, p.fp32_scales,
-        p.status);
-    encode_kernel<<<grid_for((p.element_count + 7) / 8, 256), 256, 0,
-                    stream>>>(p.values, p.element_count, p.block_shift,
-                              p.fp32_scales, p.codes);
-    if (p.scale_codes == nullptr) {
+    ScaleRecord* const records =
+        nested ? static_cast<ScaleRecord*>(p.workspace) : nullptr;
+    if (!nested) {
+        launch_fill(reinterpret_cast<float*>(p.status), 0.0F, 1, stream);
+    }
+    const unsigned groups =
+        grid_for(p.element_count, kPackValues, kMaxRecords);
+    const auto kernel =
+        p.block_shift > 9 ? pack_kernel<true> : pack_kernel<false>;
+    kernel<<<groups, kPackThreads, 0, stream>>>(
+        p.values, p.element_count, p.block_shift,
+        reinterpret_cast<std::uintptr_t>(p.values) % 16 == 0, p.fp32_scales,
+        p.codes, records, p.status);
+    if (!nested) {
         return;
     }
-    scale_mean_kernel<<<1, kMeanThreads, 0, stream>>>(
-        p.fp32_scales, block_count, p.offset, p.status);
     const std::size_t group_count =
         (block_count + (std::size_t{1} << p.second_level_shift) - 1) >>
         p.second_level_shift;
-    scale_encode_kernel<<<grid_for(group_count, 4), 256, 0, stream>>>(
+    constexpr unsigned kEncodeGroups = 512;
+    scale_encode_kernel<<<
+        grid_for(group_count, kEncodeThreads / 64, kEncodeGroups),
+        kEncodeThreads, 0, stream>>>(
         p.fp32_scales, block_count, p.second_level_shift, group_count,
-        p.offset, p.scale_codes, p.second_level);
+        records, groups, p.offset, p.status, p.scale_codes, p.second_level);
 }
 
 }  // namespace rthip

@@ -1736,8 +1736,8 @@ rthip_status rthip_nf4_quantize(
     }
     const hipStream_t hip_stream = static_cast<hipStream_t>(stream);
     // [0]: status bits, [1]: the offset (a float): the first status word of
-    // the stream workspace, cleared by a kernel (no allocation per call).
-    // The call waits for the stream below, so it cannot be captured.
+    // the stream workspace (no allocation per call).  The call waits for the
+    // stream below, so it cannot be captured.
     rthip::WorkspaceLease lease;
     if (const hipError_t error =
             rthip::lease_stream_workspace(hip_stream, &lease);
@@ -1746,8 +1746,8 @@ rthip_status rthip_nf4_quantize(
     }
     unsigned* const words = reinterpret_cast<unsigned*>(lease.status_words());
     unsigned host_words[2] = {0U, 0U};
-    rthip::launch_fill(reinterpret_cast<float*>(words), 0.0F, 2, hip_stream);
     problem.status = words;
+    problem.workspace = lease.data();
     problem.offset = reinterpret_cast<float*>(words + 1);
     rthip::launch_quantize(problem, hip_stream);
     hipError_t error = hipGetLastError();

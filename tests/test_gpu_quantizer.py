@@ -1,0 +1,90 @@
+"""The quantizer's single pass (riftco-transformer_amd/csrc/nf4_quantize.hip):
+codes at the exact turning points between neighbouring entries, every block
+size's way of finding its largest value, ragged ends and unaligned sources,
+and sums of scales on either side of where their order begins to matter.  All
+outputs are compared bit for bit with the oracle's."""
+import numpy as np
+import pytest
+
+import helpers
+
+pytestmark = pytest.mark.gpu
+
+CODEBOOK = np.array([
+    -1.0, -0.6961928009986877, -0.5250730514526367, -0.39491748809814453,
+    -0.28444138169288635, -0.18477343022823334, -0.09105003625154495, 0.0,
+    0.07958029955625534, 0.16093020141124725, 0.24611230194568634,
+    0.33791524171829224, 0.44070982933044434, 0.5626170039176941,
+    0.7229568362236023, 1.0], dtype=np.float32)
+
+
+def check(gpu, oracle, device_dense, dense, block, nested, second=32):
+    want = oracle.quantize(dense, block, nested, second)
+    got = gpu.quantize_weight(device_dense, block, nested, second)
+    assert np.array_equal(got.codes.cpu().numpy(), want.codes)
+    primary = got.primary_scales.cpu().numpy()
+    if not nested:
+        helpers.assert_bit_equal(primary, want.fp32_scales)
+        return
+    assert np.array_equal(primary, want.scale_codes)
+    helpers.assert_bit_equal(got.secondary_scales.cpu().numpy(),
+                             want.second_level)
+    helpers.assert_bit_equal(np.float32(got.offset), np.float32(want.offset))
+
+
+@pytest.mark.parametrize("scale", [1.0, 0.02, 3.0e38, 2.0e-38, 1.0e-44])
+def test_codes_at_the_turning_points(gpu, oracle, scale):
+    """64 neighbouring floats around every midpoint, and around the entries,
+    each in a block whose largest value is the scale."""
+    import torch
+    centres = np.concatenate([
+        CODEBOOK, (CODEBOOK[1:] + CODEBOOK[:-1]) * np.float32(0.5)])
+    rows = []
+    for centre in centres * np.float32(scale):
+        value = np.float32(centre)
+        for _ in range(32):
+            value = np.nextafter(value, np.float32(-np.inf))
+        for _ in range(64):
+            rows.append(value)
+            value = np.nextafter(value, np.float32(np.inf))
+    limit = np.float32(scale)
+    values = np.clip(np.array(rows, dtype=np.float32), -limit, limit)
+    dense = values.reshape(-1, 31)
+    dense = np.concatenate(
+        [dense, np.full((dense.shape[0], 1), limit, np.float32)], axis=1)
+    check(gpu, oracle, torch.from_numpy(dense).cuda(), dense, 32, False)
+
+
+@pytest.mark.parametrize("nested", [False, True])
+@pytest.mark.parametrize("block", [32, 64, 128, 512, 1024, 4096])
+@pytest.mark.parametrize("count", [1, 37, 4095, 4097, 20485])
+def test_block_sizes_ends_and_alignment(gpu, oracle, block, nested, count):
+    import torch
+    dense = helpers.normal(911, (1, count), 0.02)
+    dense[0, : min(count, 100)] = 0.0
+    buffer = torch.zeros(count + 4, device="cuda")
+    for shift in (0, 1, 2):
+        view = buffer[shift:shift + count]
+        view.copy_(torch.from_numpy(dense[0]))
+        check(gpu, oracle, view.view(1, count), dense, block, nested)
+
+
+def test_more_tiles_than_workgroups(gpu, oracle):
+    import torch
+    dense = helpers.normal(912, (1031, 8193), 0.02)  # 2063 tiles of 4096
+    check(gpu, oracle, torch.from_numpy(dense).cuda(), dense, 1024, True, 256)
+
+
+@pytest.mark.parametrize("exponents", [5, 24, 25, 26, 27, 28, 29, 40])
+def test_order_of_the_scales_sum(gpu, oracle, exponents):
+    """Sixteen large scales and many small odd ones: from 2^53 units in the
+    last place of the smallest on, a double no longer holds every sum."""
+    import torch
+    rng = np.random.default_rng(913)
+    blocks = 3000
+    scales = np.float32(1.0) + rng.random(blocks).astype(np.float32)
+    scales[rng.choice(blocks, 16, replace=False)] *= np.float32(
+        2.0 ** exponents)
+    dense = np.zeros((blocks, 32), dtype=np.float32)
+    dense[:, 5] = scales
+    check(gpu, oracle, torch.from_numpy(dense).cuda(), dense, 32, True)
