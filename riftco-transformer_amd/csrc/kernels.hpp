@@ -40,11 +40,24 @@ struct LinearProblem {
 void launch_generic_forward(const LinearProblem& problem, hipStream_t stream);
 hipError_t launch_generic_input_backward(const LinearProblem& problem,
                                          hipStream_t stream);
+// result[e] = sum over chunks, ascending, of partial[chunk][e] (+ the adapter
+// term): the end of an input backward whose weight rows were cut into chunks.
+void launch_backward_sum(const LinearProblem& problem, const float* partial,
+                         std::size_t chunks, hipStream_t stream);
 void launch_dequantize(const Nf4WeightView& weight, float* out,
                        std::size_t element_count, unsigned block_shift,
                        hipStream_t stream);
 void launch_fill(float* out, float value, std::size_t count,
                  hipStream_t stream);
+
+// nf4_ragged.hip -- both directions, any widths from one step of the
+// contraction on, any row count, on the fp32 matrix instruction;
+// launch_generic_* take it where it applies.
+bool ragged_forward_supports(const LinearProblem& problem);
+bool ragged_input_backward_supports(const LinearProblem& problem);
+void launch_ragged_forward(const LinearProblem& problem, hipStream_t stream);
+hipError_t launch_ragged_input_backward(const LinearProblem& problem,
+                                        hipStream_t stream);
 
 // nf4_gemv.hip -- forward only, small row counts.
 constexpr std::size_t kGemvMaxRows = 4;

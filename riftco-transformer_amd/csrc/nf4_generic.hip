@@ -254,6 +254,10 @@ unsigned grid_for(std::size_t work_items, std::size_t items_per_block) {
 }  // namespace
 
 void launch_generic_forward(const LinearProblem& p, hipStream_t stream) {
+    if (ragged_forward_supports(p)) {
+        launch_ragged_forward(p, stream);
+        return;
+    }
     const std::size_t items =
         (p.rows + kRowGroup - 1) / kRowGroup * p.output_width;
     generic_forward_kernel<<<grid_for(items, 4), 256, 0, stream>>>(
@@ -263,6 +267,9 @@ void launch_generic_forward(const LinearProblem& p, hipStream_t stream) {
 
 hipError_t launch_generic_input_backward(const LinearProblem& p,
                                          hipStream_t stream) {
+    if (ragged_input_backward_supports(p)) {
+        return launch_ragged_input_backward(p, stream);
+    }
     const std::size_t tiles =
         (p.input_width + kBackwardColumns - 1) / kBackwardColumns;
     const std::size_t groups = (p.rows + kRowGroup - 1) / kRowGroup;
@@ -300,12 +307,16 @@ hipError_t launch_generic_input_backward(const LinearProblem& p,
         p.activations, p.weight, target, p.rows, p.input_width,
         p.output_width, p.block_shift, chunk_rows, p.lora);
     if (chunks > 1) {
-        const std::size_t elements = p.rows * p.input_width;
-        generic_backward_sum_kernel<<<grid_for(elements, 256), 256, 0,
-                                      stream>>>(
-            target, p.result, elements, chunks, p.input_width, p.lora);
+        launch_backward_sum(p, target, chunks, stream);
     }
     return hipSuccess;
+}
+
+void launch_backward_sum(const LinearProblem& p, const float* partial,
+                         std::size_t chunks, hipStream_t stream) {
+    const std::size_t elements = p.rows * p.input_width;
+    generic_backward_sum_kernel<<<grid_for(elements, 256), 256, 0, stream>>>(
+        partial, p.result, elements, chunks, p.input_width, p.lora);
 }
 
 void launch_dequantize(const Nf4WeightView& weight, float* out,

@@ -1,0 +1,648 @@
+// Packed NF4 products whose widths are multiples of nothing: rows of the
+// weight that start at any nibble, quantisation blocks that straddle rows.
+//
+//   forward         y [M, O] = x  [M, I] * deq(W)^T     (contract over I)
+//   input backward  dx[M, I] = dy [M, O] * deq(W)       (contract over O)
+//
+// restating reference_quantized_linear_forward / _input_backward
+// (src/core/backend/nn/quantized_linear/reference/operations.cpp:49-115).
+//
+// Eight or sixteen neighbouring weights are one lane's share of a step,
+// wherever they start: the 32-bit words around their codes, shifted into place,
+// and the two scales that they can meet.  They go straight into the fp32 matrix
+// instruction (16 x 16 x 4), whose contraction order is free as long as both
+// operands keep it, so that nothing passes through LDS before the final sum of
+// the wavefronts.
+//
+// What bounds it: the address units of the vector memory path.  Lanes of a load
+// lie in sixteen rows, i.e. in sixteen cache lines or more, and the fp32 matrix
+// instruction (157 TFLOP/s) takes about half the time.  Hence long spans per
+// lane forward: with eight weights instead of sixteen, twice as many code and
+// scale loads per weight, 16 rows of 4097 x 4095 took 29 us; a third step of
+// loads in flight made it 40.  One wavefront per output column with a byte and
+// a scale load per weight (nf4_generic.hip) against this kernel, fp32 scales,
+// forward / input backward:
+//     4097 x 4095, 1 row        22 -> 17     59 -> 22 us
+//     4097 x 4095, 16 rows     209 -> 23    185 -> 24
+//     4097 x 4095, 64 rows     661 -> 67    703 -> 48
+//     4097 x 4095, 2048 rows 22400 -> 1120  9390 -> 825
+//     301 x 777, 300 rows       37 -> 14     49 -> 17
+// and the error against sums in 64 bits 1.5e-7 -> 1.1...1.4e-7 / 1.6...2.0e-7
+// -> 1.1...1.4e-7 at 4097 x 4095.
+
+#include "kernels.hpp"
+#include "nf4_decode.hpp"
+#include "scale_reader.hpp"
+
+#include <algorithm>
+
+namespace rthip {
+namespace {
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+constexpr unsigned kRowBlock = 16;  // rows of x or dy per matrix instruction
+// neighbouring weights of a lane, forward and backward
+constexpr unsigned kForwardSpan = 16;
+constexpr unsigned kBackwardSpan = 8;
+
+struct RaggedTables {
+    float levels[16];
+    float factors[256];  // nested scales: (code - 128) / 127
+};
+
+template <bool kDoubleQuantized>
+__device__ __forceinline__ void fill_tables(RaggedTables& tables) {
+    load_codebook_to_lds(tables.levels);
+    if constexpr (kDoubleQuantized) {
+        if (threadIdx.x < 256) {
+            tables.factors[threadIdx.x] =
+                static_cast<float>(static_cast<int>(threadIdx.x) - 128) /
+                127.0F;
+        }
+    }
+    __syncthreads();
+}
+
+// kSpan neighbouring weights as they were loaded: the words around their
+// codes, and the scales of the first and the last of them (a block has at
+// least 32 weights).
+template <unsigned kSpan>
+struct LoadedSpan {
+    static constexpr unsigned kWords = kSpan / 8 + 1;
+    unsigned words[kWords];
+    LoadedScale first;
+    LoadedScale last;
+};
+
+template <unsigned kSpan, bool kDoubleQuantized>
+class SpanReader {
+public:
+    __device__ __forceinline__ SpanReader(const Nf4WeightView& weight,
+                                          unsigned weights,
+                                          unsigned block_shift)
+        : scales_(weight, weights, block_shift),
+          block_mask_((1U << block_shift) - 1U) {
+        // Whole words through the descriptor; the one to three bytes that may
+        // follow them are read one by one and no byte past them is.
+        const unsigned bytes = (weights + 1U) / 2U;
+        words_ = bytes / 4U;
+        codes_ = make_buffer(weight.codes, words_ * 4U);
+        const __amdgpu_buffer_rsrc_t all = make_buffer(weight.codes, bytes);
+        tail_ = 0U;
+#pragma unroll
+        for (unsigned byte = 0; byte < 3; ++byte) {
+            tail_ |= static_cast<unsigned>(__builtin_amdgcn_raw_buffer_load_b8(
+                         all, words_ * 4U + byte, 0, 0))
+                     << (8U * byte);
+        }
+    }
+    // Requests the weights [flat, flat + kSpan); codes and scales past the
+    // last weight are zeros or another weight's.
+    __device__ __forceinline__ LoadedSpan<kSpan> load(unsigned flat) const {
+        const unsigned offset = flat / 8U * 4U;
+        LoadedSpan<kSpan> out;
+#pragma unroll
+        for (unsigned i = 0; i < LoadedSpan<kSpan>::kWords; ++i) {
+            out.words[i] = __builtin_amdgcn_raw_buffer_load_b32(
+                codes_, offset + 4U * i, 0, 0);
+        }
+        out.first = scales_.load(flat, true);
+        out.last = scales_.load(flat + kSpan - 1U, true);
+        return out;
+    }
+    // The weights: level times scale, one rounded multiply.
+    __device__ __forceinline__ void decode(const LoadedSpan<kSpan>& loaded,
+                                           unsigned flat,
+                                           const RaggedTables& tables,
+                                           float (&out)[kSpan]) const {
+#pragma clang fp contract(off)
+        constexpr unsigned kWords = LoadedSpan<kSpan>::kWords;
+        unsigned words[kWords];
+#pragma unroll
+        for (unsigned i = 0; i < kWords; ++i) {
+            words[i] = flat / 8U + i == words_ ? tail_ : loaded.words[i];
+        }
+        const float first = scales_.decode(loaded.first, tables.factors);
+        const float last = scales_.decode(loaded.last, tables.factors);
+        // weights left in the first one's block
+        const unsigned left = block_mask_ + 1U - (flat & block_mask_);
+#pragma unroll
+        for (unsigned i = 0; i + 1 < kWords; ++i) {
+            const unsigned codes = __builtin_amdgcn_alignbit(
+                words[i + 1], words[i], flat % 8U * 4U);
+#pragma unroll
+            for (unsigned n = 0; n < 8; ++n) {
+                const float level = tables.levels[(codes >> (4U * n)) & 0xFU];
+                const float scale = 8 * i + n < left ? first : last;
+                out[8 * i + n] = level * scale;
+            }
+        }
+    }
+
+private:
+    ScaleReader<kDoubleQuantized> scales_;
+    __amdgpu_buffer_rsrc_t codes_;
+    unsigned block_mask_;
+    unsigned words_;
+    unsigned tail_;
+};
+
+// Four neighbouring floats (a row may start at any float, which the wide load
+// allows).
+__device__ __forceinline__ floatx4 load_four(__amdgpu_buffer_rsrc_t buffer,
+                                             unsigned lane, unsigned offset) {
+    return __builtin_bit_cast(
+        floatx4,
+        __builtin_amdgcn_raw_buffer_load_b128(buffer, lane, offset, 0));
+}
+
+// Forward.  A workgroup owns sixteen columns of y and kGroups blocks of
+// sixteen rows; its wavefronts take the steps of 64 contraction values in
+// turn.  Lane l holds contraction values [16 * (l / 16), + 16) of column l % 16
+// and of row l % 16 of every block.  grid = (columns / 16, rows / (16 *
+// kGroups)).  The contraction has at least 64 values; where it is not a
+// multiple of 64, the last step covers the last 64 of them and takes those
+// that the step before it had as zeros: every load is a whole one, without a
+// branch, and the next steps' stay in flight past it.
+//
+// Few enough registers for two workgroups on a compute unit: 4097 columns are
+// 257 workgroups, and one left over from a first round would cost as much as
+// the round.
+template <int kGroups>
+struct ForwardShape {
+    static constexpr unsigned kWaves = 8;
+    // steps of loads in flight
+    static constexpr int kStages = kGroups <= 2 ? 2 : 1;
+    // sums of a step per block of rows at a time
+    static constexpr int kChains = kGroups == 1 ? 4 : 1;
+    // wavefronts per SIMD: two workgroups
+    static constexpr unsigned kResident = 2 * kWaves / 4;
+};
+constexpr unsigned kForwardStep = 4 * kForwardSpan;
+constexpr unsigned kForwardColumns = 16;
+
+template <int kGroups, bool kDoubleQuantized>
+__global__ __launch_bounds__(ForwardShape<kGroups>::kWaves * 64,
+                             ForwardShape<kGroups>::kResident)
+void ragged_forward_kernel(const float* __restrict__ x, Nf4WeightView weight,
+                           const float* __restrict__ bias,
+                           float* __restrict__ y, unsigned rows,
+                           unsigned input_width, unsigned output_width,
+                           unsigned block_shift, LoraEpilogue lora) {
+    constexpr unsigned kWaves = ForwardShape<kGroups>::kWaves;
+    constexpr int kStages = ForwardShape<kGroups>::kStages;
+    constexpr int kChains = ForwardShape<kGroups>::kChains;
+    __shared__ RaggedTables tables;
+    __shared__ floatx4 parts[kWaves][64];
+
+    const unsigned lane = threadIdx.x % 64;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const unsigned quarter = lane / 16;
+    const unsigned first_row = blockIdx.y * (kRowBlock * kGroups);
+    const unsigned first_column = blockIdx.x * kForwardColumns;
+    const SpanReader<kForwardSpan, kDoubleQuantized> spans(
+        weight, input_width * output_width, block_shift);
+    // (columns past the last one repeat it and are not written)
+    const unsigned flat0 =
+        min(first_column + lane % 16, output_width - 1U) * input_width +
+        kForwardSpan * quarter;
+    // rows past the last one are past the extent: zeros
+    const __amdgpu_buffer_rsrc_t input = make_buffer(
+        x + static_cast<std::size_t>(first_row) * input_width,
+        min(rows - first_row, kRowBlock * kGroups) * input_width *
+            static_cast<unsigned>(sizeof(float)));
+    const unsigned lane_input = (lane % 16 * input_width + kForwardSpan * quarter) *
+                                static_cast<unsigned>(sizeof(float));
+    const unsigned group_bytes =
+        kRowBlock * input_width * static_cast<unsigned>(sizeof(float));
+
+    struct Stage {
+        LoadedSpan<kForwardSpan> span;
+        floatx4 x[kGroups][kForwardSpan / 4];
+    };
+    Stage stages[kStages];
+    floatx4 total[kGroups];
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) {
+        total[g] = floatx4{0.0F, 0.0F, 0.0F, 0.0F};
+    }
+    const unsigned steps = (input_width + kForwardStep - 1U) / kForwardStep;
+    const unsigned overlap = steps * kForwardStep - input_width;
+    // (past the last step: that one again, which is not used)
+    const auto first_value = [&](unsigned step) {
+        return min(step * kForwardStep, input_width - kForwardStep);
+    };
+    const auto load = [&](Stage& stage, unsigned step) {
+        const unsigned k0 = first_value(step);
+        stage.span = spans.load(flat0 + k0);
+        const unsigned offset = k0 * static_cast<unsigned>(sizeof(float));
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) {
+#pragma unroll
+            for (unsigned h = 0; h < kForwardSpan / 4; ++h) {
+                stage.x[g][h] = load_four(
+                    input, lane_input + g * group_bytes + 16U * h, offset);
+            }
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < kStages; ++s) {
+        load(stages[s], wave + s * kWaves);
+    }
+    const auto multiply = [&](Stage& stage, unsigned step) {
+        float w[kForwardSpan];
+        spans.decode(stage.span, flat0 + first_value(step), tables, w);
+        if (step + 1U == steps && overlap != 0U) {  // uniform
+#pragma unroll
+            for (unsigned n = 0; n < kForwardSpan; ++n) {
+                const bool had = kForwardSpan * quarter + n < overlap;
+                w[n] = had ? 0.0F : w[n];
+#pragma unroll
+                for (int g = 0; g < kGroups; ++g) {
+                    stage.x[g][n / 4][n % 4] =
+                        had ? 0.0F : stage.x[g][n / 4][n % 4];
+                }
+            }
+        }
+        // Sums of sixteen products, added in pairs where the registers allow
+        // it: the rounding stays below that of one sum per lane.
+        const floatx4 zero{0.0F, 0.0F, 0.0F, 0.0F};
+#pragma unroll
+        for (int first = 0; first < 4; first += kChains) {
+            floatx4 sums[kGroups][kChains];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                for (int g = 0; g < kGroups; ++g) {
+#pragma unroll
+                    for (int c = 0; c < kChains; ++c) {
+                        sums[g][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            stage.x[g][first + c][e], w[4 * (first + c) + e],
+                            e == 0 ? zero : sums[g][c], 0, 0, 0);
+                    }
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g) {
+                if constexpr (kChains == 4) {
+                    sums[g][0] += sums[g][1];
+                    sums[g][2] += sums[g][3];
+                    sums[g][0] += sums[g][2];
+                }
+                total[g] += sums[g][0];
+            }
+        }
+    };
+
+    fill_tables<kDoubleQuantized>(tables);
+    for (unsigned step = wave; step < steps; step += kStages * kWaves) {
+#pragma unroll
+        for (int s = 0; s < kStages; ++s) {
+            if (s == 0 || step + s * kWaves < steps) {  // uniform
+                multiply(stages[s], step + s * kWaves);
+            }
+            if (step + (kStages + s) * kWaves < steps) {  // uniform
+                load(stages[s], step + (kStages + s) * kWaves);
+            }
+        }
+    }
+
+    // The wavefronts' sums, added in pairs.  Element e of lane l is row 4 *
+    // (l / 16) + e, column l % 16 of the block.
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) {
+        parts[wave][lane] = total[g];
+        __syncthreads();
+        if (threadIdx.x < 256) {
+            const unsigned m = threadIdx.x / 16;
+            const unsigned n = threadIdx.x % 16;
+            const unsigned row = first_row + kRowBlock * g + m;
+            const unsigned column = first_column + n;
+            if (row < rows && column < output_width) {
+                const float* const source =
+                    reinterpret_cast<const float*>(
+                        &parts[0][m / 4 * 16 + n]) + m % 4;
+                float sums[kWaves];
+#pragma unroll
+                for (unsigned w = 0; w < kWaves; ++w) {
+                    sums[w] = source[w * 256];
+                }
+#pragma unroll
+                for (unsigned half = kWaves / 2; half != 0; half /= 2) {
+#pragma unroll
+                    for (unsigned w = 0; w < half; ++w) {
+                        sums[w] += sums[w + half];
+                    }
+                }
+                float value = sums[0];
+                if (bias != nullptr) {
+                    value += bias[column];
+                }
+                if (lora.reduced != nullptr) {
+                    value += lora_term(lora, row, column);
+                }
+                y[static_cast<std::size_t>(row) * output_width + column] =
+                    value;
+            }
+        }
+        if (g + 1 < kGroups) {
+            __syncthreads();
+        }
+    }
+}
+
+// Input backward.  A workgroup owns 128 columns of dx, kGroups blocks of
+// sixteen rows and one chunk of the weight rows; its eight wavefronts take the
+// chunk's steps of sixteen weight rows in turn.  Lane l holds the eight
+// columns [8 * (l % 16), + 8) of the weight rows 4 * (l / 16) + j, j < 4:
+// weight t of each is the operand of a product of its own, whose sixteen
+// columns lie eight apart, and no transpose is needed.  The weight has at
+// least sixteen rows, and the last step is a whole one as above.  grid = (columns / 128,
+// chunks, rows / (16 * kGroups)); with one chunk the sums go to dx, otherwise
+// to `target`, [chunk][rows][input_width].
+constexpr unsigned kBackwardWaves = 8;
+constexpr unsigned kBackwardStep = 16;
+constexpr unsigned kBackwardColumns = 16 * kBackwardSpan;
+constexpr int kBackwardStages = 2;
+
+template <int kGroups, bool kDoubleQuantized>
+__global__ __launch_bounds__(kBackwardWaves * 64, kGroups == 1 && !kDoubleQuantized ? 4 : 2)
+void ragged_input_backward_kernel(
+    const float* __restrict__ dy, Nf4WeightView weight,
+    float* __restrict__ target, unsigned rows, unsigned input_width,
+    unsigned output_width, unsigned block_shift, unsigned chunk_rows,
+    LoraEpilogue lora
+) {
+    __shared__ RaggedTables tables;
+    __shared__ floatx4 parts[kBackwardWaves][4][64];
+
+    const unsigned lane = threadIdx.x % 64;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const unsigned quarter = lane / 16;
+    const unsigned first_row = blockIdx.z * (kRowBlock * kGroups);
+    const unsigned first_column = blockIdx.x * kBackwardColumns;
+    const unsigned column = first_column + kBackwardSpan * (lane % 16);
+    const unsigned begin = blockIdx.y * chunk_rows;
+    const unsigned end = min(begin + chunk_rows, output_width);
+    const SpanReader<kBackwardSpan, kDoubleQuantized> spans(
+        weight, input_width * output_width, block_shift);
+    const __amdgpu_buffer_rsrc_t upstream = make_buffer(
+        dy + static_cast<std::size_t>(first_row) * output_width,
+        min(rows - first_row, kRowBlock * kGroups) * output_width *
+            static_cast<unsigned>(sizeof(float)));
+    const unsigned lane_upstream =
+        (lane % 16 * output_width + 4U * quarter) *
+        static_cast<unsigned>(sizeof(float));
+    const unsigned group_bytes =
+        kRowBlock * output_width * static_cast<unsigned>(sizeof(float));
+
+    struct Stage {
+        LoadedSpan<kBackwardSpan> span[4];
+        floatx4 dy[kGroups];
+    };
+    Stage stages[kBackwardStages];
+    floatx4 total[kGroups][kBackwardSpan];
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) {
+#pragma unroll
+        for (unsigned t = 0; t < kBackwardSpan; ++t) {
+            total[g][t] = floatx4{0.0F, 0.0F, 0.0F, 0.0F};
+        }
+    }
+    // (past the last step: that one again, which is not used)
+    const auto first_weight_row = [&](unsigned o) {
+        return min(o, output_width - kBackwardStep);
+    };
+    // (columns past a row's end are other weights or zeros, and not written)
+    const auto flat_of = [&](unsigned o0, int j) {
+        return (o0 + 4U * quarter + j) * input_width + column;
+    };
+    const auto load = [&](Stage& stage, unsigned o) {
+        const unsigned o0 = first_weight_row(o);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            stage.span[j] = spans.load(flat_of(o0, j));
+        }
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) {
+            stage.dy[g] = load_four(
+                upstream, lane_upstream + g * group_bytes,
+                o0 * static_cast<unsigned>(sizeof(float)));
+        }
+    };
+    constexpr unsigned kRound = kBackwardWaves * kBackwardStep;
+    const unsigned start = begin + wave * kBackwardStep;
+#pragma unroll
+    for (int s = 0; s < kBackwardStages; ++s) {
+        load(stages[s], start + s * kRound);
+    }
+    fill_tables<kDoubleQuantized>(tables);
+    const auto multiply = [&](Stage& stage, unsigned o) {
+        const unsigned o0 = first_weight_row(o);
+        const unsigned overlap = o - o0;
+        if (overlap != 0U) {  // uniform
+#pragma unroll
+            for (unsigned j = 0; j < 4; ++j) {
+#pragma unroll
+                for (int g = 0; g < kGroups; ++g) {
+                    stage.dy[g][j] = 4U * quarter + j < overlap
+                                         ? 0.0F
+                                         : stage.dy[g][j];
+                }
+            }
+        }
+        const floatx4 zero{0.0F, 0.0F, 0.0F, 0.0F};
+        floatx4 sums[kGroups][kBackwardSpan];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float w[kBackwardSpan];
+            spans.decode(stage.span[j], flat_of(o0, j), tables, w);
+            if (overlap != 0U) {  // uniform
+#pragma unroll
+                for (unsigned t = 0; t < kBackwardSpan; ++t) {
+                    w[t] = 4U * quarter + j < overlap ? 0.0F : w[t];
+                }
+            }
+#pragma unroll
+            for (unsigned t = 0; t < kBackwardSpan; ++t) {
+#pragma unroll
+                for (int g = 0; g < kGroups; ++g) {
+                    sums[g][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        stage.dy[g][j], w[t], j == 0 ? zero : sums[g][t], 0, 0,
+                        0);
+                }
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) {
+#pragma unroll
+            for (unsigned t = 0; t < kBackwardSpan; ++t) {
+                total[g][t] += sums[g][t];
+            }
+        }
+    };
+
+    for (unsigned o = start; o < end; o += kBackwardStages * kRound) {
+#pragma unroll
+        for (int s = 0; s < kBackwardStages; ++s) {
+            if (s == 0 || o + s * kRound < end) {  // uniform
+                multiply(stages[s], o + s * kRound);
+            }
+            if (o + (kBackwardStages + s) * kRound < end) {  // uniform
+                load(stages[s], o + (kBackwardStages + s) * kRound);
+            }
+        }
+    }
+
+    // The wavefronts' sums, in their order, four of a lane's columns at a
+    // time.
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) {
+#pragma unroll
+        for (unsigned half = 0; half < 2; ++half) {
+            if (g + half != 0) {
+                __syncthreads();
+            }
+#pragma unroll
+            for (unsigned t = 0; t < 4; ++t) {
+                parts[wave][t][lane] = total[g][4 * half + t];
+            }
+            __syncthreads();
+            if (threadIdx.x < 256) {
+                // thread -> (lane of the sums, its column t)
+                const unsigned t = threadIdx.x % 4;
+                const unsigned from = threadIdx.x / 4;
+                floatx4 sum{0.0F, 0.0F, 0.0F, 0.0F};
+#pragma unroll
+                for (unsigned w = 0; w < kBackwardWaves; ++w) {
+                    sum += parts[w][t][from];
+                }
+                const unsigned out_column =
+                    first_column + kBackwardSpan * (from % 16) + 4 * half + t;
+#pragma unroll
+                for (unsigned e = 0; e < 4; ++e) {
+                    const unsigned row =
+                        first_row + kRowBlock * g + from / 16 * 4 + e;
+                    if (row < rows && out_column < input_width) {
+                        float value = sum[e];
+                        if (gridDim.y == 1 && lora.reduced != nullptr) {
+                            value += lora_term(lora, row, out_column);
+                        }
+                        target[(static_cast<std::size_t>(blockIdx.y) * rows +
+                                row) * input_width + out_column] = value;
+                    }
+                }
+            }
+        }
+    }
+}
+
+template <int kGroups, bool kDoubleQuantized>
+void launch_forward(const LinearProblem& p, hipStream_t stream) {
+    const unsigned rows = static_cast<unsigned>(p.rows);
+    const unsigned input_width = static_cast<unsigned>(p.input_width);
+    const unsigned output_width = static_cast<unsigned>(p.output_width);
+    constexpr unsigned kRows = kRowBlock * kGroups;
+    const dim3 grid((output_width + kForwardColumns - 1U) / kForwardColumns,
+                    (rows + kRows - 1U) / kRows);
+    ragged_forward_kernel<kGroups, kDoubleQuantized>
+        <<<grid, ForwardShape<kGroups>::kWaves * 64, 0, stream>>>(
+            p.activations, p.weight, p.bias, p.result, rows, input_width,
+            output_width, p.block_shift, p.lora);
+}
+
+template <int kGroups, bool kDoubleQuantized>
+hipError_t launch_backward(const LinearProblem& p, hipStream_t stream) {
+    const unsigned rows = static_cast<unsigned>(p.rows);
+    const unsigned input_width = static_cast<unsigned>(p.input_width);
+    const unsigned output_width = static_cast<unsigned>(p.output_width);
+    constexpr unsigned kRows = kRowBlock * kGroups;
+    constexpr unsigned kRound = kBackwardWaves * kBackwardStep;
+    const unsigned tiles =
+        (input_width + kBackwardColumns - 1U) / kBackwardColumns;
+    const unsigned groups = (rows + kRows - 1U) / kRows;
+    // Chunks of weight rows, in rounds of a workgroup's steps, until there are
+    // two workgroups per compute unit, as far as the workspace holds their
+    // sums.
+    constexpr unsigned kWantedBlocks = 512;
+    const std::size_t per_chunk =
+        std::size_t{rows} * input_width * sizeof(float);
+    const std::size_t blocks = std::size_t{tiles} * groups;
+    std::size_t chunks = std::min<std::size_t>(
+        {(kWantedBlocks + blocks - 1) / blocks,
+         (output_width + kRound - 1U) / kRound,
+         kStreamWorkspaceBytes / per_chunk});
+    chunks = std::max<std::size_t>(chunks, 1);
+    const unsigned rounds = (output_width + kRound - 1U) / kRound;
+    const unsigned chunk_rows =
+        (rounds + static_cast<unsigned>(chunks) - 1U) /
+        static_cast<unsigned>(chunks) * kRound;
+    chunks = (output_width + chunk_rows - 1U) / chunk_rows;
+    float* target = p.result;
+    WorkspaceLease lease;  // held until both launches are enqueued
+    if (chunks > 1) {
+        if (const hipError_t status = lease_stream_workspace(stream, &lease);
+            status != hipSuccess) {
+            return status;
+        }
+        target = lease.data();
+    }
+    const dim3 grid(tiles, static_cast<unsigned>(chunks), groups);
+    ragged_input_backward_kernel<kGroups, kDoubleQuantized>
+        <<<grid, kBackwardWaves * 64, 0, stream>>>(
+            p.activations, p.weight, target, rows, input_width, output_width,
+            p.block_shift, chunk_rows, p.lora);
+    if (chunks > 1) {
+        launch_backward_sum(p, target, chunks, stream);
+    }
+    return hipSuccess;
+}
+
+bool common_supports(const LinearProblem& p) {
+    constexpr std::size_t kWidthLimit = std::size_t{1} << 22;
+    return p.input_width < kWidthLimit && p.output_width < kWidthLimit &&
+           // 32-bit flat indices, some weights past the last one included
+           p.input_width * p.output_width < (std::size_t{1} << 31) &&
+           // the grid's second and third dimensions
+           p.rows <= std::size_t{65535} * kRowBlock &&
+           // words of codes
+           reinterpret_cast<std::uintptr_t>(p.weight.codes) % 4 == 0;
+}
+
+}  // namespace
+
+bool ragged_forward_supports(const LinearProblem& p) {
+    return p.input_width >= kForwardStep && common_supports(p);
+}
+
+bool ragged_input_backward_supports(const LinearProblem& p) {
+    return p.output_width >= kBackwardStep && common_supports(p);
+}
+
+void launch_ragged_forward(const LinearProblem& p, hipStream_t stream) {
+    const bool nested = p.weight.encoding != 0;
+    if (p.rows <= kRowBlock) {
+        nested ? launch_forward<1, true>(p, stream)
+               : launch_forward<1, false>(p, stream);
+    } else if (p.rows <= 2 * kRowBlock) {
+        nested ? launch_forward<2, true>(p, stream)
+               : launch_forward<2, false>(p, stream);
+    } else {
+        nested ? launch_forward<4, true>(p, stream)
+               : launch_forward<4, false>(p, stream);
+    }
+}
+
+hipError_t launch_ragged_input_backward(const LinearProblem& p,
+                                        hipStream_t stream) {
+    const bool nested = p.weight.encoding != 0;
+    if (p.rows <= kRowBlock) {
+        return nested ? launch_backward<1, true>(p, stream)
+                      : launch_backward<1, false>(p, stream);
+    }
+    return nested ? launch_backward<2, true>(p, stream)
+                  : launch_backward<2, false>(p, stream);
+}
+
+}  // namespace rthip

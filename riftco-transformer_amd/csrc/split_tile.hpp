@@ -36,6 +36,7 @@
 
 #include "gemv_shared.hpp"
 #include "kernels.hpp"
+#include "scale_reader.hpp"
 #include "tile_plan.hpp"
 
 #include <cstddef>
@@ -57,7 +58,6 @@ constexpr int kTileN = 128;       // output columns per workgroup
 constexpr unsigned kFragmentBytes = 1024;  // 32 rows x 16 contraction values
 constexpr unsigned kUnit = 32;  // contraction values per TilePlan unit
 constexpr unsigned kFlushValues = 256;  // contraction values per accumulation
-constexpr unsigned kOutside = 0xFFFFFFFFU;  // past every descriptor's extent
 
 // A pointer that is the same in every lane, in scalar registers: the compiler
 // takes quotients and 64-bit products to the vector unit and would read a

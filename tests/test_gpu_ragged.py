@@ -1,0 +1,96 @@
+"""The packed products at widths that are multiples of nothing
+(riftco-transformer_amd/csrc/nf4_ragged.hip): rows that start at either nibble
+of a byte and at any byte of a word, blocks that straddle rows, codes whose
+last word is not whole.
+
+Bounds.  Products are exact before their fp32 additions, and at most 36 of
+those follow one another on a value before it meets the other wavefronts'
+sums; the suite's bar of 1e-5 of a K-normalised output leaves a factor of ten.
+A row with a single one in it meets no rounding at all."""
+import numpy as np
+import pytest
+
+import helpers
+
+pytestmark = pytest.mark.gpu
+
+TOLERANCE = 1.0e-5
+
+
+def packed(oracle, gpu, out_w, in_w, block, nested, seed):
+    weight = oracle.quantize(helpers.normal(seed, (out_w, in_w), 0.02), block,
+                             nested, 32)
+    device = gpu.upload_weight(
+        out_w, in_w, block, weight.codes, fp32_scales=weight.fp32_scales,
+        scale_codes=weight.scale_codes, second_level=weight.second_level,
+        second_level_block=weight.second_level_block, offset=weight.offset)
+    return device, oracle.dequantize(weight)
+
+
+def run(gpu, function, activations, weight, package):
+    import torch
+    out = function(torch.from_numpy(activations).cuda(), weight,
+                   algorithm=package.ALGORITHM_GENERIC)
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("nested", [False, True])
+@pytest.mark.parametrize("rows,out_w,in_w,block", [
+    (1, 1, 1, 32),            # one nibble, no whole word
+    (2, 3, 7, 32),            # one block over all rows; 11 bytes
+    (3, 15, 63, 32),          # shorter than a step, both directions
+    (3, 16, 64, 64),          # one step, both directions
+    (1, 17, 65, 32),          # a column past the sixteen, a value past a step
+    (16, 129, 127, 64),       # a column past the backward's 128
+    (17, 33, 1025, 32),       # two blocks of rows
+    (33, 255, 513, 4096),     # four blocks of rows; one block over eight rows
+    (65, 130, 259, 128),      # a second workgroup of rows
+    (130, 515, 1031, 64),     # rows past two workgroups, two rounds of steps
+    (5, 2051, 301, 64),       # backward in chunks
+])
+def test_any_widths(gpu, package, oracle, rows, out_w, in_w, block, nested):
+    weight, dense = packed(oracle, gpu, out_w, in_w, block, nested, 921)
+    unit = helpers.rms(dense)
+    for function, width, product in (
+            (gpu.linear_forward, in_w, helpers.exact_forward),
+            (gpu.linear_input_backward, out_w, helpers.exact_input_backward)):
+        values = helpers.normal(922, (rows, width), 1.0)
+        got = run(gpu, function, values, weight, package)
+        error = helpers.normalized_error(got, product(values, dense), width,
+                                         1.0, unit)
+        assert error <= TOLERANCE, f"{function.__name__}: {error:.3g}"
+
+
+@pytest.mark.parametrize("nested", [False, True])
+@pytest.mark.parametrize("out_w,in_w,block", [(37, 45, 32), (45, 38, 64)])
+def test_single_ones_return_the_weight(gpu, package, oracle, out_w, in_w,
+                                       block, nested):
+    weight, dense = packed(oracle, gpu, out_w, in_w, block, nested, 923)
+    forward = run(gpu, gpu.linear_forward, np.eye(in_w, dtype=np.float32),
+                  weight, package)
+    backward = run(gpu, gpu.linear_input_backward,
+                   np.eye(out_w, dtype=np.float32), weight, package)
+    # (adding zero turns the code for zero's sign positive in both)
+    helpers.assert_bit_equal(forward + 0.0, dense.T + 0.0)
+    helpers.assert_bit_equal(backward + 0.0, dense + 0.0)
+
+
+def test_infinite_values_stay_in_their_rows(gpu, package, oracle):
+    """The last step's padding meets neither the next row's values nor the
+    weights past a row's end."""
+    weight, dense = packed(oracle, gpu, 67, 35, 32, False, 924)
+    for function, width, product in (
+            (gpu.linear_forward, 35, helpers.exact_forward),
+            (gpu.linear_input_backward, 67, helpers.exact_input_backward)):
+        values = helpers.normal(925, (20, width), 1.0)
+        values[4, 0] = np.inf
+        values[9, width - 1] = np.nan
+        got = run(gpu, function, values, weight, package)
+        with np.errstate(invalid="ignore"):
+            exact = product(values, dense).astype(np.float32)
+        assert np.array_equal(np.isfinite(got), np.isfinite(exact))
+        plain = np.setdiff1d(np.arange(20), [4, 9])
+        error = helpers.normalized_error(got[plain], exact[plain], width, 1.0,
+                                         helpers.rms(dense))
+        assert error <= TOLERANCE
