@@ -375,8 +375,9 @@ rthip_status rthip_nf4_lora_linear_input_backward_with(
  * and up to 192 in three parts where output_width >= 2 * input_width).
  * Where the register-resident kernel takes the rows, 81...128 are one launch
  * of it and 129...224 two, 128 rows and the rest.  Larger row counts that end
- * 1...64 rows past a multiple of 128 run as a tiled launch for the whole
- * 128-row tiles and a small-batch launch for the rest, in both directions.
+ * 1...64 rows past whole tiles of 256 rows run as a tiled launch for those and
+ * a small-batch launch for the rest, in both directions, if there is enough work
+ * for such tiles; so do a few rows past tiles of 128.
  * The family of the first part is reported. */
 rthip_status rthip_nf4_select_algorithm(
     int32_t direction, uint64_t rows, uint64_t input_width,

@@ -573,6 +573,11 @@ bool mfma_forward_supports(const LinearProblem& p) {
     return common_supports(p) && p.input_width % 32 == 0;
 }
 
+bool mfma_takes_tall_tiles(const LinearProblem& p, bool forward) {
+    return use_tall_tiles(1, p.rows, forward ? p.input_width : p.output_width,
+                          forward ? p.output_width : p.input_width);
+}
+
 hipError_t launch_mfma_forward(const LinearProblem& p, hipStream_t stream) {
     return launch<false>(p, stream);
 }

@@ -353,33 +353,57 @@ bool backward_small_split(const rthip::LinearProblem& problem,
     return true;
 }
 
-// The tiled kernel works in row tiles of 128.  A row count that ends up to 64
-// rows past a multiple of 128 would pay a whole tile row for them (11008 x
-// 4096: ~93 us, whatever the count); AUTO gives those last rows to the
-// small-batch families instead, after the tiled launch for the rows before
-// them.  Measured, forward / input backward, nested scales: 272 rows of
-// 11008 x 4096 320 -> 243 / 315 -> 237 us, 320 rows 319 -> 283 / 318 -> 273
-// us, 2080 rows 1682 -> 1618 / 1649 -> 1594 us; 4096 x 4096 at 272 rows
-// 144 -> 116 / 138 -> 112 us; with 94 rows left over both ways are even, so
-// from 65 on the tile row stays.
+// A row count that ends up to 64 rows past a whole number of tall tiles (256
+// rows, split_tile.hpp) would take the tiled kernel's square tiles for all of
+// its rows, and a tile row of its own for the last ones; AUTO gives those to
+// the small-batch families instead, after a tall launch for the rows before
+// them.  One launch -> two, fp32 scales, forward / input backward: 272 rows of
+// 11008 x 4096 212 -> 156 / 211 -> 152 us, 320 rows 213 -> 199 / 213 -> 187,
+// 2064 rows 1101 -> 930 / 1053 -> 907; 4096 x 4096 at 272 rows 89 -> 71 / 88
+// -> 73 us.  Where the rows before them would run in square tiles too there is
+// nothing to gain (1024 x 4096 at 320 rows 33 -> 36 / 37 -> 48 us), nor past an
+// odd number of 128-row tiles, which the tall tiles pad to one more (4096 x
+// 11008 at 192 rows 118 -> 149 / 122 -> 162 us).
+//
+// Few rows are an exception, as they cost little by themselves.  Forward, what
+// the streaming family takes (257 rows of 1024 x 4096 34 -> 30 us, of 3072 x
+// 3072 56 -> 50, 386 rows of 11008 x 4096 232 -> 219; 512 x 1024 has lost by
+// then, 21 -> 23); backward only past one 128-row tile and on larger weights
+// (4096 x 11008 at 129 rows 112 -> 96 us, 1024 x 4096 28 -> 35).  Either way up
+// to sixteen rows past whole tall tiles of larger weights (2048 x 4096 at 257
+// rows 52 -> 42 / 52 -> 49, at 272 rows 51 -> 50 / 52 -> 50).
 constexpr std::size_t kTileRows = 128;
+constexpr std::size_t kTallTileRows = 256;
 constexpr std::size_t kTailSplitMaxRows = 64;
+constexpr std::size_t kShortTailRows = 16;
 bool tail_split(const rthip::LinearProblem& problem, bool forward,
                 RowSplit* split) {
     const auto select = forward ? select_forward : select_input_backward;
     const std::size_t tail = problem.rows % kTileRows;
-    if (problem.rows <= kTileRows || tail == 0 || tail > kTailSplitMaxRows ||
+    const std::size_t head = problem.rows - tail;
+    if (head == 0 || tail == 0 || tail > kTailSplitMaxRows ||
         select(problem) != RTHIP_NF4_ALGORITHM_MFMA) {
         return false;
     }
     split->count = 2;
-    split->part[0] = row_part(problem, 0, problem.rows - tail, forward);
-    split->part[1] = row_part(problem, problem.rows - tail, tail, forward);
+    split->part[0] = row_part(problem, 0, head, forward);
+    split->part[1] = row_part(problem, head, tail, forward);
     split->family[0] = select(split->part[0]);
     split->family[1] = select(split->part[1]);
-    return split->family[0] == RTHIP_NF4_ALGORITHM_MFMA &&
-           (small_batch_family(split->family[1]) ||
-            split->family[1] == RTHIP_NF4_ALGORITHM_GEMV);
+    const bool streamed = split->family[1] == RTHIP_NF4_ALGORITHM_GEMV;
+    if (split->family[0] != RTHIP_NF4_ALGORITHM_MFMA ||
+        !(streamed || small_batch_family(split->family[1]))) {
+        return false;
+    }
+    const std::size_t weights = problem.output_width * problem.input_width;
+    const bool large = weights >= (std::size_t{1} << 23);
+    if (streamed && (forward ? head == kTileRows ||
+                                   weights >= (std::size_t{1} << 22)
+                             : head == kTileRows && large)) {
+        return true;
+    }
+    return (large && tail <= kShortTailRows && head % kTallTileRows == 0) ||
+           rthip::mfma_takes_tall_tiles(split->part[0], forward);
 }
 // Two to four rows of x against weight rows too wide for the GEMV to hold
 // that many rows of x in registers (from 16384 weights on) run as two GEMV

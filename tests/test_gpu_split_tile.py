@@ -150,3 +150,44 @@ def test_dense_matmul_of_infinite_values(gpu):
                                rtol=4.0e-7)
     plain = np.isfinite(exact) & (np.abs(exact) < 1.0e3)
     assert np.abs(got - exact)[plain].max() <= TOLERANCE * np.sqrt(70)
+
+
+@pytest.mark.parametrize("rows,head", [
+    (129, 128),    # one square tile row and the streaming families' rows
+    (133, 133),    # too many rows for those: one launch
+    (192, 192),
+    (257, 256),    # whole tall tiles and the rest
+    (320, 256),
+    (321, 321),    # more than 64 rows left over
+    (400, 400),    # an odd number of 128-row tiles before the rest
+])
+@pytest.mark.parametrize("out_w,in_w,tall", [
+    (4224, 4160, True),
+    (1056, 1088, False),     # 256 rows would not run in tall tiles
+])
+def test_rows_past_whole_tiles(gpu, package, oracle, rows, head, out_w, in_w,
+                               tall):
+    """The automatic choice runs the rows before `head` and the rest as calls
+    of their own would, bit for bit, and stays within the bar."""
+    import torch
+    weight, dense = packed(package, oracle, gpu, out_w, in_w, 64, True, 911)
+    exact = torch.from_numpy(dense).cuda().double()
+    unit = helpers.rms(dense)
+    for function, width, right in (
+            (gpu.linear_forward, in_w, exact.T.contiguous()),
+            (gpu.linear_input_backward, out_w, exact)):
+        if not tall and (head == 256 or
+                         function is gpu.linear_input_backward):
+            head = rows
+        values = torch.from_numpy(
+            helpers.normal(912, (rows, width), 1.0)).cuda()
+        got = function(values, weight)
+        parts = [function(values[:head].contiguous(), weight,
+                          algorithm=package.ALGORITHM_MFMA)]
+        if head < rows:
+            parts.append(function(values[head:].contiguous(), weight))
+        assert torch.equal(got, torch.cat(parts)), function.__name__
+        error = helpers.normalized_error(
+            got.cpu().numpy(), (values.double() @ right).cpu().numpy(), width,
+            1.0, unit)
+        assert error <= TOLERANCE, f"{function.__name__}: {error:.3g}"
