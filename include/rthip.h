@@ -79,7 +79,8 @@ enum {
      * walked row by row as it lies in memory, a lane owning sixteen of its
      * columns, products on the 4x4x1 matrix instruction */
     RTHIP_NF4_ALGORITHM_GEMV = 2,
-    /* LDS-tiled fp32 MFMA GEMM with dequantisation fused into the tile load */
+    /* LDS-tiled MFMA GEMM (fp32 products on the bf16 matrix instruction) with
+     * dequantisation fused into the tile load */
     RTHIP_NF4_ALGORITHM_MFMA = 3,
     /* small batches (up to 64 rows): weights decoded straight into MFMA
      * operands, no LDS tile.  Forward: a slab kernel over the contraction;
